@@ -521,6 +521,18 @@ __device__ __forceinline__ void lm_tile16(const LmTileArgs& a, int prod, int p, 
     }
     if (g.kcount) K = min(K, (min(K, *g.kcount) + BK - 1) / BK * BK);
   }
+  // A product's K piece (ksplit): stages [ks0, ks0 + nk) of the tile's K / BK. Pieces are
+  // the outer index, so the tiles that share a piece's slabs run together.
+  int ks0 = 0, nk = K / BK, piece = 0;
+  if constexpr (!TL) {
+    if (g.ksplit > 1) {
+      const int tiles = ntt * nvt, per = (nk + g.ksplit - 1) / g.ksplit;
+      piece = p / tiles;
+      p -= piece * tiles;
+      ks0 = piece * per;
+      nk = max(min(per, nk - ks0), 0);
+    }
+  }
   int tm, tn;
   if (FWD && lm_fwd_vocab_groups(ntt, K))
     lm_tile_of_vgroups(p, ntt, nvt, kLmFwdVocabGroup, tm, tn);
@@ -559,7 +571,7 @@ __device__ __forceinline__ void lm_tile16(const LmTileArgs& a, int prod, int p, 
   auto issue = [&](int st, int buf) {
     char* base = smem + buf * kBuf;
     const uint32_t koff = static_cast<uint32_t>(st) * ROWB;
-    const uint32_t kofw = static_cast<uint32_t>(st) * wstage;
+    const uint32_t kofw = static_cast<uint32_t>(ks0 + st) * wstage;
 #pragma unroll
     for (int q = 0; q < QN; ++q) {
       __builtin_amdgcn_raw_ptr_buffer_load_lds(rw, LM_LDS(base + (QN * wave + q) * 1024), 16, dofw[q] + kofw, 0, 0,
@@ -604,7 +616,7 @@ __device__ __forceinline__ void lm_tile16(const LmTileArgs& a, int prod, int p, 
 #pragma unroll
       for (int j = 0; j < NJ16; ++j)
         bt[kk][j] =
-            __builtin_bit_cast(bf16x8, buf_ld16<false>(rt, roff[j] + static_cast<uint32_t>(KS16 * st + kk) * 1024u));
+            __builtin_bit_cast(bf16x8, buf_ld16<false>(rt, roff[j] + static_cast<uint32_t>(KS16 * (ks0 + st) + kk) * 1024u));
     }
   };
   f32x4 acc[NI16][NJ16];
@@ -651,7 +663,6 @@ __device__ __forceinline__ void lm_tile16(const LmTileArgs& a, int prod, int p, 
   // MFMAs. At the barrier of iteration kb the loads issued after stage kb + 1's DMA are
   // the ring reloads of (kb, 1) and (kb + 1, 0) (none in the forward): vmcnt(2 NJ16),
   // or vmcnt(0), leaves only those in flight.
-  const int nk = K / BK;
   // The forward's policy tiles also write W^T [H, ldwt] (the dhidden product's token
   // operand, fragment-major) from the W slabs they hold: stage st of vocab tile tn by
   // token tile st % ntt, so each stage is written once and every token tile writes
@@ -894,7 +905,7 @@ __device__ __forceinline__ void lm_tile16(const LmTileArgs& a, int prod, int p, 
     // (i, r) each 16-lane group writes 16 consecutive floats of one row per token block,
     // and the wave's four token blocks follow each other, so each row's 256 bytes are
     // written by four consecutive stores (whole cache lines before any eviction).
-    float* C = g.C;
+    float* C = g.C + piece * g.cstride;
     const int ldc = g.ldc, accumulate = g.accumulate;
     const int n0 = m0 + wt * TW + (lane & 15);
 #pragma unroll
@@ -921,7 +932,7 @@ __device__ __forceinline__ int lm_total_tiles(const LmTileArgs& a, int prod) {
   if constexpr (MODE == kLmGemm) {
     const LmTileArgs::Gemm& g = a.gemm[prod];
     const int V = g.vcount ? min(g.V, *g.vcount) : g.V;
-    return g.ntt * ((V + BV - 1) / BV);
+    return g.ntt * ((V + BV - 1) / BV) * max(g.ksplit, 1);
   } else {
     const int N = min(a.N, *a.count);
     return ((N + BT - 1) / BT) * a.nvt;
@@ -1234,18 +1245,40 @@ __global__ void __launch_bounds__(256) lm_gather_rows_kernel(const u32x4* src, u
   for (int i = threadIdx.x; i < nv; i += 256) d[i] = s[i];
 }
 
-__global__ void __launch_bounds__(256) lm_scatter_rows_kernel(const u32x4* src, u32x4* dst, const int* cidx, int H) {
+// Element i of the sum of nsplit pieces, in order, eight loads in flight at a time.
+__device__ __forceinline__ f32x4 lm_piece_sum(const f32x4* src, int64_t i, int nsplit, int64_t stride4) {
+  f32x4 acc = src[i];
+  int s = 1;
+  for (; s + 8 <= nsplit; s += 8) {
+    f32x4 v[8];
+#pragma unroll
+    for (int q = 0; q < 8; ++q) v[q] = src[i + (s + q) * stride4];
+#pragma unroll
+    for (int q = 0; q < 8; ++q) acc += v[q];
+  }
+  for (; s < nsplit; ++s) acc += src[i + s * stride4];
+  return acc;
+}
+
+__global__ void __launch_bounds__(256) lm_scatter_rows_kernel(const f32x4* src, int nsplit, int64_t stride4, f32x4* dst,
+                                                              const int* cidx, int H) {
   const int t = blockIdx.x;
   const int nv = H / 4;  // 16-byte vectors per f32 row
   const int c = cidx[t];
-  u32x4* d = dst + static_cast<int64_t>(t) * nv;
+  f32x4* d = dst + static_cast<int64_t>(t) * nv;
   if (c >= 0) {
-    const u32x4* s = src + static_cast<int64_t>(c) * nv;
-    for (int i = threadIdx.x; i < nv; i += 256) d[i] = s[i];
+    const int64_t r = static_cast<int64_t>(c) * nv;
+    for (int i = threadIdx.x; i < nv; i += 256) d[i] = lm_piece_sum(src, r + i, nsplit, stride4);
   } else {
-    const u32x4 z = {0u, 0u, 0u, 0u};
+    const f32x4 z = {0.f, 0.f, 0.f, 0.f};
     for (int i = threadIdx.x; i < nv; i += 256) d[i] = z;
   }
+}
+
+__global__ void __launch_bounds__(256) lm_sum_parts_kernel(const f32x4* src, int nsplit, int64_t stride4, f32x4* dst,
+                                                           int64_t n4, int64_t row4, const int* count) {
+  const int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+  if (i < n4 && (!count || i < *count * row4)) dst[i] = lm_piece_sum(src, i, nsplit, stride4);
 }
 
 // bf16 transpose through LDS, 64 x 64 tiles: 16-byte loads along source rows and
@@ -1359,7 +1392,7 @@ hipError_t launch_lm_gemms(const LmTileArgs::Gemm* g, int n_gemm, bool k_major_a
   for (int p = 0; p < a.n_gemm; ++p) {
     a.gemm[p] = g[p];
     a.gemm[p].group_m = lm_group_m(kLmGemm, g[p].ntt);
-    grid += g[p].ntt * g[p].nvt;
+    grid += g[p].ntt * g[p].nvt * (g[p].ksplit > 1 ? g[p].ksplit : 1);
   }
   if (grid <= 0) return hipSuccess;
   const bool frag = a.n_gemm > 0 && a.gemm[0].a_frag;
@@ -1371,6 +1404,7 @@ hipError_t launch_lm_gemms(const LmTileArgs::Gemm* g, int n_gemm, bool k_major_a
     // 64-deep blocks, a tile's K extent (ldb / 64 blocks of 32 KB) in 32-bit offsets.
     if (q.b_tiled && (!frag || q.ldb % 64 != 0 || q.K > q.ldb || static_cast<int64_t>(q.ldb / 64) * 32768 >= (int64_t{1} << 32)))
       return hipErrorInvalidValue;
+    if (q.ksplit > 1 && !frag) return hipErrorInvalidValue;
   }
   if (frag) return launch_tiles_mode<kLmGemm, false, false, true>(a, grid, st);
   if (!k_major_a) return launch_tiles_mode<kLmGemm, false, false>(a, grid, st);
@@ -1428,10 +1462,44 @@ hipError_t launch_lm_gather_rows(const void* src, void* dst, const int* live, co
   return hipGetLastError();
 }
 
-hipError_t launch_lm_scatter_rows(const float* src, float* dst, const int* cidx, int N, int H, hipStream_t st) {
-  lm_scatter_rows_kernel<<<dim3(N), dim3(256), 0, st>>>(reinterpret_cast<const u32x4*>(src),
-                                                        reinterpret_cast<u32x4*>(dst), cidx, H);
+hipError_t launch_lm_scatter_rows(const float* src, int nsplit, int64_t stride, float* dst, const int* cidx, int N,
+                                  int H, hipStream_t st) {
+  lm_scatter_rows_kernel<<<dim3(N), dim3(256), 0, st>>>(reinterpret_cast<const f32x4*>(src), nsplit, stride / 4,
+                                                        reinterpret_cast<f32x4*>(dst), cidx, H);
   return hipGetLastError();
+}
+
+hipError_t launch_lm_sum_parts(const float* src, int nsplit, int64_t stride, float* dst, int64_t n, int64_t rows,
+                               const int* count, hipStream_t st) {
+  if (n <= 0 || rows <= 0) return hipSuccess;
+  lm_sum_parts_kernel<<<dim3(static_cast<unsigned>((n / 4 + 255) / 256)), dim3(256), 0, st>>>(
+      reinterpret_cast<const f32x4*>(src), nsplit, stride / 4, reinterpret_cast<f32x4*>(dst), n / 4, n / rows / 4, count);
+  return hipGetLastError();
+}
+
+// The cached backward's dhidden has few, long tiles (one per 256 tokens x 256 hidden
+// columns, K = the vocabulary: 2374 stages at V = 151,936), dW many short ones, so with
+// few tokens a handful of CUs ran dhidden for milliseconds after dW was done: 288 live
+// tokens at H = 896 took 2.89 ms for the launch, 8 CUs busy. A product whose tile is longer
+// than half of a CU's even share of the launch is therefore cut along K into pieces of
+// half that share (the share counts every token, and about half of them are live, so a
+// piece is then a CU's live share), at least 16 stages (below that a piece's f32 tile
+// costs more than its products). Each piece stores its own f32 partial tile, and the pieces
+// are added in order, so results stay deterministic. Whole calls, ms, before and with
+// pieces of 1/2, 1/4, 1/8 and 1/16 of the share (tokens x H x V):
+//    64 x  256 x 151936  3.70 |  .254  .253  .254  .251
+//   512 x  896 x 151936  3.39 |  .740  .745  .785  .800
+//  1024 x 4096 x 151936  5.30 |  3.12  3.09  3.12  3.17
+//  2048 x 2048 x  50257  1.70 |  1.02  1.03  1.07  1.14
+//  4096 x  896 x 151936  4.60 |  2.60  2.63  2.65  2.70
+// 16384 x  256 x   1000  .319 |  .165  .166  .165  .165   (here dW is the long one)
+// Configuration 5 (its dhidden tiles are an eighth of the share) stays whole.
+int lm_ksplit(int64_t tiles, int64_t stages, int64_t other) {
+  constexpr int64_t kCus = 256, kMin = 16;
+  const int64_t share = (tiles * stages + other) / kCus;   // stages per CU, evenly dealt
+  if (tiles <= 0 || 2 * stages <= share) return 1;
+  const int64_t piece = share / 2 > kMin ? share / 2 : kMin;
+  return static_cast<int>((stages + piece - 1) / piece);
 }
 
 hipError_t launch_lm_zero(float* dst, int64_t n, hipStream_t st) {

@@ -78,6 +78,9 @@ struct LmTileArgs {
     int ldc;            //   C[t * ldc + v] with transpose_c (then V % 4 == 0)
     int transpose_c;
     int accumulate;     // 1: C += product, 0: C = product
+    int ksplit;         // (a_frag only) 0 or 1, or the K pieces of each tile: piece s sums its
+    int64_t cstride;    //   K range into C + s * cstride (pieces past K write zeros); the
+                        //   caller adds the pieces up
     int ntt, nvt;       // tiles over N and over V (nvt at the largest V)
     int group_m;        // set by launch_lm_gemms
   } gemm[2];
@@ -174,8 +177,18 @@ hipError_t launch_lm_compact(const LmCompactArgs& a, hipStream_t st);
 // dst[c, :] = src[live[c], :] for c < *count <= n (bf16 rows of H elements, H % 64 == 0).
 hipError_t launch_lm_gather_rows(const void* src, void* dst, const int* live, const int* count, int n, int H,
                                  hipStream_t st);
-// dst[t, :] = cidx[t] >= 0 ? src[cidx[t], :] : 0 for t < N (f32 rows of H elements).
-hipError_t launch_lm_scatter_rows(const float* src, float* dst, const int* cidx, int N, int H, hipStream_t st);
+// dst[t, :] = cidx[t] >= 0 ? src[cidx[t], :] : 0 for t < N (f32 rows of H elements); src
+// is the sum of nsplit pieces `stride` elements apart, added in order.
+hipError_t launch_lm_scatter_rows(const float* src, int nsplit, int64_t stride, float* dst, const int* cidx, int N,
+                                  int H, hipStream_t st);
+// dst[i] = sum over s < nsplit of src[s * stride + i], in order, for i < n, or with count
+// for i < *count * (n / rows) (rows whole rows of n / rows elements; multiples of 4).
+// dst may be src.
+hipError_t launch_lm_sum_parts(const float* src, int nsplit, int64_t stride, float* dst, int64_t n, int64_t rows,
+                               const int* count, hipStream_t st);
+// K pieces per tile for the fragment-major products: `tiles` tiles of `stages` 64-deep
+// stages each, in a launch whose other product adds `other` tile-stages (at all tokens).
+int lm_ksplit(int64_t tiles, int64_t stages, int64_t other);
 hipError_t launch_lm_zero(float* dst, int64_t n, hipStream_t st);
 hipError_t launch_lm_tiles(int mode, const LmTileArgs& a, hipStream_t st);
 // One launch of one or two products (n_gemm = 1 or 2; fields per LmTileArgs::Gemm,

@@ -170,7 +170,16 @@ int run_lm(pcp_ctx* ctx, const pcp_lmhead_args* a) {
   // that one block writes or one tile reads on the same HBM channels).
   const int64_t ldt_max = (N + 63) / 64 * 64 + ((N + 63) / 64 * 64 % 256 == 0 ? 64 : 0);
   const size_t o_ht = a->dweight ? take(2 * static_cast<size_t>(H) * ldt_max) : 0;
-  const size_t o_dhc = want_dy ? take(4 * static_cast<size_t>(N) * H) : 0;
+  // The cached backward's products in K pieces (lm_ksplit): dhidden's pieces are compact
+  // [N, H] buffers one after the other, dW's [V, H] ones (at most 2 x 256 CUs' worth of
+  // 256 x 256 f32 tiles in all, 134 MB). A tile's prologue and epilogue count as four stages.
+  const int64_t nht = (H + kLmTileT - 1) / kLmTileT, ntk = (N + kLmTileV - 1) / kLmTileV;
+  const int64_t sd = (V + 63) / 64 + 4, sw = (N + 63) / 64 + 4;
+  const bool may_split = bwd && a->vocab_chunk == 0;
+  const int split_d = may_split && want_dy ? lm_ksplit(ntk * nht, sd, a->dweight ? nvt * nht * sw : 0) : 1;
+  const int split_w = may_split && a->dweight ? lm_ksplit(nvt * nht, sw, want_dy ? ntk * nht * sd : 0) : 1;
+  const size_t o_dhc = want_dy ? take(4 * static_cast<size_t>(N) * H * split_d) : 0;
+  const size_t o_dwp = split_w > 1 ? take(4 * static_cast<size_t>(V) * H * split_w) : 0;
   const size_t o_rstd = norm ? take(4 * N) : 0;
   const size_t o_gpart = a->dnorm_weight ? take(4 * static_cast<size_t>(kLmNormSlices) * H) : 0;
   rc = ensure_scratch(ctx, off);
@@ -457,6 +466,8 @@ int run_lm(pcp_ctx* ctx, const pcp_lmhead_args* a) {
         d.ntt = static_cast<int>((H + kLmTileT - 1) / kLmTileT);
         d.C = dhc;
         d.ldc = static_cast<int>(H);
+        d.ksplit = split_d;
+        d.cstride = N * H;
       }
       if (a->dweight) {
         // dW[v][h] = sum_t D^T[v][t] * hidden^T[h][t].
@@ -473,8 +484,10 @@ int run_lm(pcp_ctx* ctx, const pcp_lmhead_args* a) {
         d.kcount = cnt;
         d.nvt = static_cast<int>((V + kLmTileV - 1) / kLmTileV);
         d.ntt = static_cast<int>((H + kLmTileT - 1) / kLmTileT);
-        d.C = a->dweight;
+        d.C = split_w > 1 ? F(o_dwp) : a->dweight;
         d.ldc = static_cast<int>(H);
+        d.ksplit = split_w;
+        d.cstride = V * H;
       }
       const bool timed = ctx->prof_on && ctx->prof_used < static_cast<int>(ctx->prof_start.size());
       if (timed && (e = hipEventRecord(ctx->prof_start[ctx->prof_used], st)) != hipSuccess)
@@ -483,6 +496,9 @@ int run_lm(pcp_ctx* ctx, const pcp_lmhead_args* a) {
         return hip_fail(ctx, e, "dhidden / dweight products");
       if (timed && (e = hipEventRecord(ctx->prof_stop[ctx->prof_used++], st)) != hipSuccess)
         return hip_fail(ctx, e, "hipEventRecord");
+      if (split_w > 1 &&
+          (e = launch_lm_sum_parts(F(o_dwp), split_w, V * H, a->dweight, V * H, V, nullptr, st)) != hipSuccess)
+        return hip_fail(ctx, e, "adding the dweight pieces");
     } else {
       if (a->dweight && (e = chunk_frag ? launch_lm_transpose_frag(tr, st) : launch_lm_transpose(tr, st)) != hipSuccess)
         return hip_fail(ctx, e, "transposing hidden rows");
@@ -556,13 +572,16 @@ int run_lm(pcp_ctx* ctx, const pcp_lmhead_args* a) {
           return hip_fail(ctx, e, "dhidden / dweight products");
       }
     }
+    const int pieces = cached ? split_d : 1;   // of the compact dhidden
     if (norm && want_dy) {
+      if (pieces > 1 && (e = launch_lm_sum_parts(dhc, pieces, N * H, dhc, N * H, N, cnt, st)) != hipSuccess)
+        return hip_fail(ctx, e, "adding the dhidden pieces");
       const LmNormBwdArgs nb{dhc, static_cast<const uint16_t*>(a->hidden_states), a->norm_weight, F(o_rstd),
                              I(o_cidx), I(o_live), N, static_cast<int>(H), cnt, a->dhidden,
                              a->dnorm_weight ? F(o_gpart) : nullptr, a->dnorm_weight};
       if ((e = launch_lm_norm_bwd(nb, st)) != hipSuccess) return hip_fail(ctx, e, "final norm backward");
-    } else if (!norm && a->dhidden && (e = launch_lm_scatter_rows(dhc, a->dhidden, I(o_cidx), static_cast<int>(N),
-                                                         static_cast<int>(H), st)) != hipSuccess) {
+    } else if (!norm && a->dhidden && (e = launch_lm_scatter_rows(dhc, pieces, N * H, a->dhidden, I(o_cidx),
+                                                                     static_cast<int>(N), static_cast<int>(H), st)) != hipSuccess) {
       return hip_fail(ctx, e, "scattering dhidden rows");
     }
   }

@@ -203,6 +203,27 @@ def test_lmhead_small_vs_oracle(shape, mode):
     check_grads(out, *grad_bounds(c, L, lse, r, mode, old, cached=chunk == 0))
 
 
+# Products cut along K (lm_ksplit): dhidden in 17 pieces, the last of one stage (V = 16,400
+# is 257 stages of 64), and in 2 with a ragged vocabulary tail; dW in 7 pieces of which the
+# live tokens (8 of 6,000) fill one stage of the first, so six are empty; one live token.
+SPLIT = [(1, 40, 64, 16400, 1, [33]), (2, 130, 320, 1090, 2, [130, 129]), (2, 3000, 64, 300, 2, [5, 3]),
+         (2, 3000, 128, 130, 1, [1, 0])]
+
+
+@pytest.mark.parametrize("exact", [False, True], ids=["cached", "exact"])
+@pytest.mark.parametrize("shape", SPLIT, ids=lambda s: f"S{s[0]}T{s[1]}H{s[2]}V{s[3]}")
+def test_lmhead_split_products_vs_oracle(shape, exact):
+    S, T, H, V, G, lengths = shape
+    c = make_case(S, T, H, V, G, seed=S * 977 + T + V, lengths=lengths)
+    mode = LossMode.GRPO_CLIP_KL
+    L, lse, rlse, old, r = oracle_case(c, mode)
+    out = run_device(c, mode, old, exact_bf16=exact)
+    check_forward(c, out, L, lse, rlse, r, mode)
+    check_grads(out, *grad_bounds(c, L, lse, r, mode, old, cached=not exact))
+    again = run_device(c, mode, old, exact_bf16=exact)
+    assert torch.equal(out.dhidden, again.dhidden) and torch.equal(out.dweight, again.dweight)
+
+
 @pytest.mark.parametrize("shape", [s for s in SMALL if s[5] > 0], ids=lambda s: f"S{s[0]}T{s[1]}H{s[2]}V{s[3]}c{s[5]}")
 def test_lmhead_small_low_memory_chunks_vs_oracle(shape):
     """The chunked backward's low-memory form (K-major operands read with LDS transpose
