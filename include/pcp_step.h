@@ -57,6 +57,11 @@ typedef struct {
 
 int pcp_grad_stats_compute(pcp_ctx* ctx, const float* grad, int64_t n, int accumulate, pcp_grad_stats* stats,
                            void* stream);
+/* The same over n_tensors tensors at once (grads[i] on the device, counts[i] elements; the
+ * two arrays are host memory, read during the call): one pass of launches and one wait for
+ * all of them, where a loop over pcp_grad_stats_compute waits for each tensor. */
+int pcp_grad_stats_compute_many(pcp_ctx* ctx, int n_tensors, const float* const* grads, const int64_t* counts,
+                                int accumulate, pcp_grad_stats* stats, void* stream);
 
 /* ---- Nesterov optimizer on HBM (src/optimizers/nesterov.zig) ---------------------- */
 typedef enum {

@@ -164,6 +164,8 @@ SIGNATURES = {
     "pcp_mfma_peak": (_I, [_VP, _I, _I, _I, ctypes.c_uint32, _VP, _VP, _VP]),
     "pcp_pack_rollouts": (_I, [_VP, _VP, _I64, _VP, _VP, _I64, _VP, _I64, _I64, _I64, _VP, _VP, _VP]),
     "pcp_grad_stats_compute": (_I, [_VP, _VP, _I64, _I, ctypes.POINTER(GradStats), _VP]),
+    "pcp_grad_stats_compute_many": (_I, [_VP, _I, ctypes.POINTER(_VP), ctypes.POINTER(_I64), _I,
+                                         ctypes.POINTER(GradStats), _VP]),
     "pcp_nesterov_create": (_I, [_VP, _F, _F, _I, _I, ctypes.POINTER(_I64), ctypes.POINTER(_VP)]),
     "pcp_nesterov_destroy": (None, [_VP]),
     "pcp_nesterov_reset": (_I, [_VP, _VP]),

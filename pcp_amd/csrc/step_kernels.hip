@@ -101,18 +101,18 @@ struct StatsPart {
   int64_t inf_count;
 };
 
-constexpr int kStatsBlocks = 2048;
-
-__device__ __forceinline__ void stats_add(StatsPart& s, float g) {
-  if (__builtin_isnan(g)) {
-    s.nan_count += 1;
-  } else if (__builtin_isinf(g)) {
-    s.inf_count += 1;
-  } else {
-    s.sumsq += static_cast<double>(g) * static_cast<double>(g);
-    s.max_abs = fmaxf(s.max_abs, fabsf(g));
-  }
-}
+// Several tensors in one launch: tensor t's chunks of kStatsChunk elements are chunks
+// [first[t], first[t + 1]) of the launch. The table travels in the kernel's arguments
+// (2.6 KB), so a call needs no upload and keeps nothing.
+constexpr int kStatsTensors = 128;
+constexpr int kStatsChunk = 16384;
+constexpr int kStatsBlocks = 2048;   // per launch: eight 256-lane blocks on each of 256 CUs
+struct StatsBatch {
+  const float* g[kStatsTensors];
+  int64_t n[kStatsTensors];
+  int first[kStatsTensors + 1];
+  int tensors;
+};
 
 __device__ __forceinline__ void stats_merge(StatsPart& a, const StatsPart& b) {
   a.sumsq += b.sumsq;
@@ -121,15 +121,45 @@ __device__ __forceinline__ void stats_merge(StatsPart& a, const StatsPart& b) {
   a.inf_count += b.inf_count;
 }
 
-// Fixed-order tree over the 256 threads of a block (deterministic).
+// N elements at once: the sum's product is exact in f64, so the fma rounds as the
+// separate multiply and add would. The largest magnitude, as bits, says whether any of
+// them is not finite; only then are they counted one by one.
+template <int N>
+__device__ __forceinline__ void stats_add(StatsPart& s, const float (&x)[N]) {
+  uint32_t top = 0;
+#pragma unroll
+  for (int i = 0; i < N; ++i) top = max(top, __float_as_uint(x[i]) & 0x7fffffffu);
+  if (top < 0x7f800000u) {
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      const double d = static_cast<double>(x[i]);
+      s.sumsq = __builtin_fma(d, d, s.sumsq);
+    }
+    s.max_abs = fmaxf(s.max_abs, __uint_as_float(top));
+    return;
+  }
+  for (int i = 0; i < N; ++i) {
+    if (__builtin_isnan(x[i])) {
+      s.nan_count += 1;
+    } else if (__builtin_isinf(x[i])) {
+      s.inf_count += 1;
+    } else {
+      const double d = static_cast<double>(x[i]);
+      s.sumsq = __builtin_fma(d, d, s.sumsq);
+      s.max_abs = fmaxf(s.max_abs, fabsf(x[i]));
+    }
+  }
+}
+
+// Fixed-order tree over the NT threads of a block (deterministic).
+template <int NT>
 __device__ __forceinline__ StatsPart stats_block(StatsPart s, StatsPart* lds) {
   lds[threadIdx.x] = s;
   __syncthreads();
-  for (int w = 128; w > 0; w >>= 1) {
+  for (int w = NT / 2; w > 0; w >>= 1) {
     if (threadIdx.x < static_cast<unsigned>(w)) {
-      StatsPart o = lds[threadIdx.x + w];
       StatsPart m = lds[threadIdx.x];
-      stats_merge(m, o);
+      stats_merge(m, lds[threadIdx.x + w]);
       lds[threadIdx.x] = m;
     }
     __syncthreads();
@@ -137,36 +167,58 @@ __device__ __forceinline__ StatsPart stats_block(StatsPart s, StatsPart* lds) {
   return lds[0];
 }
 
-// Thread i of the grid reads vectors i, i + stride, ... (16-byte loads when the
-// pointer allows, else elements); one partial per block.
-__global__ void __launch_bounds__(256) stats_kernel(const float* g, int64_t n, int vec, StatsPart* parts) {
+// A gradient vector: 16 bytes at any element's address.
+typedef f32x4 f32x4_any __attribute__((aligned(4)));
+
+// HBM-bound: one read of every gradient. A block takes chunks blockIdx.x, + gridDim.x,
+// ..., eight 16-byte loads per lane in flight, and writes one partial.
+__global__ void __launch_bounds__(256) stats_kernel(StatsBatch b, StatsPart* parts) {
   __shared__ StatsPart lds[256];
   StatsPart s{0.0, 0.f, 0, 0, 0};
-  const int64_t tid = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
-  const int64_t stride = static_cast<int64_t>(gridDim.x) * 256;
-  if (vec) {
-    const int64_t n4 = n / 4;
-    const f32x4* g4 = reinterpret_cast<const f32x4*>(g);
-    for (int64_t i = tid; i < n4; i += stride) {
-      const f32x4 x = __builtin_nontemporal_load(g4 + i);
-      stats_add(s, x.x);
-      stats_add(s, x.y);
-      stats_add(s, x.z);
-      stats_add(s, x.w);
+  const int chunks = b.first[b.tensors];
+  for (int c = blockIdx.x; c < chunks; c += gridDim.x) {
+    int t = 0, hi = b.tensors;   // the tensor of chunk c: first[t] <= c < first[hi]
+    while (hi - t > 1) {
+      const int mid = (t + hi) / 2;
+      if (b.first[mid] <= c) t = mid;
+      else hi = mid;
     }
-    for (int64_t i = n4 * 4 + tid; i < n; i += stride) stats_add(s, g[i]);
-  } else {
-    for (int64_t i = tid; i < n; i += stride) stats_add(s, g[i]);
+    const int64_t e0 = static_cast<int64_t>(c - b.first[t]) * kStatsChunk;
+    const float* g = b.g[t] + e0;
+    const int n = static_cast<int>(min<int64_t>(kStatsChunk, b.n[t] - e0)), n4 = n / 4;
+    const f32x4_any* g4 = reinterpret_cast<const f32x4_any*>(g);
+    constexpr int kU = 8;
+    int i = threadIdx.x;
+    for (; i + (kU - 1) * 256 < n4; i += kU * 256) {
+      float x[4 * kU];
+#pragma unroll
+      for (int u = 0; u < kU; ++u) {
+        const f32x4 v = __builtin_nontemporal_load(g4 + i + u * 256);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) x[4 * u + k] = v[k];
+      }
+      stats_add(s, x);
+    }
+    for (; i < n4; i += 256) {
+      const f32x4 v = g4[i];
+      const float x[4] = {v[0], v[1], v[2], v[3]};
+      stats_add(s, x);
+    }
+    const int r = 4 * n4 + static_cast<int>(threadIdx.x);
+    if (r < n) {
+      const float x[1] = {g[r]};
+      stats_add(s, x);
+    }
   }
-  s = stats_block(s, lds);
+  s = stats_block<256>(s, lds);
   if (threadIdx.x == 0) parts[blockIdx.x] = s;
 }
 
-__global__ void __launch_bounds__(256) stats_final_kernel(const StatsPart* parts, int nparts, StatsPart* out) {
-  __shared__ StatsPart lds[256];
+__global__ void __launch_bounds__(1024) stats_final_kernel(const StatsPart* parts, int nparts, StatsPart* out) {
+  __shared__ StatsPart lds[1024];
   StatsPart s{0.0, 0.f, 0, 0, 0};
-  for (int i = threadIdx.x; i < nparts; i += 256) stats_merge(s, parts[i]);
-  s = stats_block(s, lds);
+  for (int i = threadIdx.x; i < nparts; i += 1024) stats_merge(s, parts[i]);
+  s = stats_block<1024>(s, lds);
   if (threadIdx.x == 0) *out = s;
 }
 
@@ -345,23 +397,53 @@ int pcp_pack_rollouts(pcp_ctx* ctx, const int64_t* prompt_tokens, int64_t n_prom
 
 int pcp_grad_stats_compute(pcp_ctx* ctx, const float* grad, int64_t n, int accumulate, pcp_grad_stats* stats,
                            void* stream) {
-  if (!stats || n < 0 || (n > 0 && !grad)) return fail(ctx, PCP_ERR_INVALID_ARG, "grad / stats is NULL or n < 0");
+  return pcp_grad_stats_compute_many(ctx, 1, &grad, &n, accumulate, stats, stream);
+}
+
+int pcp_grad_stats_compute_many(pcp_ctx* ctx, int n_tensors, const float* const* grads, const int64_t* counts,
+                                int accumulate, pcp_grad_stats* stats, void* stream) {
+  if (!stats || n_tensors < 0 || (n_tensors > 0 && (!grads || !counts)))
+    return fail(ctx, PCP_ERR_INVALID_ARG, "grads / counts / stats is NULL or n_tensors < 0");
+  int64_t chunks = 0, elements = 0;
+  for (int t = 0; t < n_tensors; ++t) {
+    if (counts[t] < 0 || (counts[t] > 0 && !grads[t]))
+      return fail(ctx, PCP_ERR_INVALID_ARG, "grad / stats is NULL or n < 0");
+    if (counts[t] > (int64_t(1) << 44) - elements) return fail(ctx, PCP_ERR_OVERFLOW, "more than 2^44 gradients");
+    elements += counts[t];
+    chunks += (counts[t] + kStatsChunk - 1) / kStatsChunk;
+  }
   if (!ctx) return fail(nullptr, PCP_ERR_INVALID_ARG, "context is NULL");
   hipError_t e = hipSetDevice(ctx->device);
   if (e != hipSuccess) return hip_fail(ctx, e, "hipSetDevice");
   hipStream_t st = static_cast<hipStream_t>(stream);
-  const size_t parts_bytes = sizeof(StatsPart) * (kStatsBlocks + 1);
-  int rc = ensure_scratch(ctx, parts_bytes);
-  if (rc != PCP_OK) return rc;
-  StatsPart* parts = static_cast<StatsPart*>(ctx->scratch);
   StatsPart h{0.0, 0.f, 0, 0, 0};
-  if (n > 0) {
-    const int vec = (reinterpret_cast<uintptr_t>(grad) & 15u) == 0;
-    const unsigned grid = grid_for(n, 256 * 16) < kStatsBlocks ? grid_for(n, 256 * 16) : kStatsBlocks;
-    stats_kernel<<<grid, 256, 0, st>>>(grad, n, vec, parts);
-    stats_final_kernel<<<1, 256, 0, st>>>(parts, static_cast<int>(grid), parts + kStatsBlocks);
+  if (elements > 0) {
+    // A launch takes up to kStatsTensors tensors and writes at most kStatsBlocks partials.
+    const int64_t launches = (n_tensors + kStatsTensors - 1) / kStatsTensors;
+    const int64_t cap = chunks < launches * kStatsBlocks ? chunks : launches * kStatsBlocks;
+    int rc = ensure_scratch(ctx, sizeof(StatsPart) * static_cast<size_t>(cap + 1));
+    if (rc != PCP_OK) return rc;
+    StatsPart* parts = static_cast<StatsPart*>(ctx->scratch);
+    int nparts = 0;
+    for (int t = 0; t < n_tensors;) {
+      StatsBatch b;
+      b.tensors = 0;
+      b.first[0] = 0;
+      for (; t < n_tensors && b.tensors < kStatsTensors; ++t) {
+        if (counts[t] == 0) continue;
+        b.g[b.tensors] = grads[t];
+        b.n[b.tensors] = counts[t];
+        b.first[b.tensors + 1] = b.first[b.tensors] + static_cast<int>((counts[t] + kStatsChunk - 1) / kStatsChunk);
+        ++b.tensors;
+      }
+      if (b.tensors == 0) break;
+      const int n = b.first[b.tensors], grid = n < kStatsBlocks ? n : kStatsBlocks;
+      stats_kernel<<<grid, 256, 0, st>>>(b, parts + nparts);
+      nparts += grid;
+    }
+    stats_final_kernel<<<1, 1024, 0, st>>>(parts, nparts, parts + cap);
     if ((e = hipGetLastError()) != hipSuccess) return hip_fail(ctx, e, "statistics launch");
-    if ((e = hipMemcpyAsync(&h, parts + kStatsBlocks, sizeof(h), hipMemcpyDeviceToHost, st)) != hipSuccess)
+    if ((e = hipMemcpyAsync(&h, parts + cap, sizeof(h), hipMemcpyDeviceToHost, st)) != hipSuccess)
       return hip_fail(ctx, e, "reading statistics");
     if ((e = hipStreamSynchronize(st)) != hipSuccess) return hip_fail(ctx, e, "hipStreamSynchronize");
   }
@@ -370,7 +452,7 @@ int pcp_grad_stats_compute(pcp_ctx* ctx, const float* grad, int64_t n, int accum
   stats->max_abs = std::fmax(stats->max_abs, h.max_abs);
   stats->nan_count += h.nan_count;
   stats->inf_count += h.inf_count;
-  stats->elements += n;
+  stats->elements += elements;
   stats->l2_norm = std::sqrt(stats->sumsq);
   return PCP_OK;
 }

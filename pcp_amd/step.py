@@ -44,11 +44,14 @@ def grad_stats(grads, *, stream=None, ctx: Context | None = None) -> dict:
     grads = [grads] if isinstance(grads, torch.Tensor) else list(grads)
     ctx = ctx or default_context(grads[0].device.index or 0)
     st = GradStats()
-    for i, g in enumerate(grads):
+    n = len(grads)
+    counts = [g.numel() for g in grads]
+    for g in grads:
         if g.dtype != torch.float32:
             raise PcpError(-2, "gradients must be f32")
-        check(lib().pcp_grad_stats_compute(ctx.handle, _ptr(g) if g.numel() else None, g.numel(), int(i > 0),
-                                           ctypes.byref(st), _stream_handle(stream)), ctx.handle)
+    ptrs = (ctypes.c_void_p * n)(*[_ptr(g) if k else None for g, k in zip(grads, counts)])
+    check(lib().pcp_grad_stats_compute_many(ctx.handle, n, ptrs, (ctypes.c_int64 * n)(*counts), 0, ctypes.byref(st),
+                                            _stream_handle(stream)), ctx.handle)
     return {"sumsq": st.sumsq, "l2_norm": st.l2_norm, "max_abs": st.max_abs, "nan_count": st.nan_count,
             "inf_count": st.inf_count, "elements": st.elements}
 

@@ -119,6 +119,24 @@ def test_grad_stats_match_oracle(offset):
     assert both["elements"] == want["elements"]
 
 
+@pytest.mark.parametrize("n_tensors", [1, 127, 128, 129, 300])
+def test_grad_stats_many_tensors_match_oracle(n_tensors):
+    """Tensors of 0, 1 and a few elements and around the 4-element vector, the lanes' 8,192-element
+    batch and the 16,384-element chunk, at every offset mod 16 bytes, around the 128 tensors of a
+    launch; the f64 sum of squares may differ by its order: 2^-52 per addition, far below 1e-12."""
+    rng = np.random.default_rng(n_tensors)
+    edges = [0, 1, 3, 5, 1023, 8191, 8192, 8193, 16383, 16384, 16385, 40000]
+    counts = [int(rng.choice(edges)) for _ in range(n_tensors - 1)] + [70001]
+    g = rng.standard_normal(sum(counts)).astype(np.float32)
+    g[rng.integers(0, g.size, 9)] = [np.nan, np.inf, -np.inf, 1e30, -1e-42, 0.0, -0.0, 3e38, np.nan]
+    got = step.grad_stats(list(t(g).split(counts)))
+    want = orc.grad_stats(g)
+    for k in ("nan_count", "inf_count", "elements", "max_abs"):
+        assert got[k] == want[k], k
+    assert abs(got["sumsq"] - want["sumsq"]) <= 1e-12 * want["sumsq"]
+    assert got["l2_norm"] == np.sqrt(got["sumsq"])
+
+
 def test_grad_stats_sum_of_squares_in_f64():
     x = np.array([1e20, 3.0, -1e20], np.float32)                         # squares overflow f32
     got = step.grad_stats(t(x))
