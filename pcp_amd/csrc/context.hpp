@@ -14,12 +14,25 @@ namespace pcp {
 struct HostStager;
 }
 
+namespace pcp {
+// What kernels hand back to the host: one pinned, coherent host page per context, written
+// by the device with plain system-scope stores and read by the host after the stream is
+// synchronised, so no call copies a result back. (An error word in device memory cost
+// every synchronous call a 4-byte hipMemcpy after its wait: see collect_device_errors.)
+struct HostPage {
+  int err[8];                      // err[i] != 0: condition 1 << i (kErr* bits) was raised
+  int b64_pad;                     // padding characters of the last base64 decode
+  alignas(64) char stats[64];      // the gradient statistics' result
+};
+}  // namespace pcp
+
 struct pcp_ctx {
   int device = 0;
   int backend = PCP_BACKEND_ROCM;
   char last_error[512] = {};      // fixed buffer: reporting an error allocates nothing
-  int* d_err = nullptr;          // device error word (kErr* bits)
-  int* d_next_row = nullptr;     // row counter of the persistent row kernel (same allocation)
+  pcp::HostPage* page = nullptr;    // host address of the page kernels report through
+  pcp::HostPage* d_page = nullptr;  // its device address
+  int* d_next_row = nullptr;     // row counter of the persistent row kernel
   void* scratch = nullptr;       // per-call work buffers, grown on demand
   size_t scratch_bytes = 0;
   // Streams holding PCP_FLAG_ASYNC work (a fixed set, so recording one allocates nothing).
@@ -88,7 +101,8 @@ inline int dtype_bytes(int dt) {
 // Make `bytes` of scratch available on ctx (grow-only; synchronises before a free).
 int ensure_scratch(pcp_ctx* ctx, size_t bytes);
 
-// After synchronising: read and clear the device error word, map it to a status.
+// After synchronising: read and clear the error slots of the context's page, map them to
+// a status.
 int collect_device_errors(pcp_ctx* ctx);
 
 // Record a stream that holds PCP_FLAG_ASYNC work for pcp_sync. When the fixed set is

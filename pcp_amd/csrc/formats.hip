@@ -124,6 +124,12 @@ __global__ void __launch_bounds__(256) b64_encode_groups_kernel(const uint8_t* s
   }
 }
 
+// One store per wave that met a bad character.
+__device__ __forceinline__ void raise_bad(uint32_t bad, int* err) {
+  const uint64_t lanes = __ballot((bad & 0x80808080u) != 0);
+  if (lanes && static_cast<int>(threadIdx.x & 63) == __builtin_ctzll(lanes)) raise_error(err, kErrBadBase64);
+}
+
 // Fast decode over whole 16-character units before the final quad (src 16-byte aligned,
 // dst 4-byte aligned): one quad load and three dword stores per lane, contiguous across
 // the wave. A character outside the alphabet sets kErrBadBase64.
@@ -154,14 +160,14 @@ __global__ void __launch_bounds__(256) b64_decode_kernel(const u32x4* __restrict
       __builtin_nontemporal_store(c, dst + 3 * i + 2);
     }
   }
-  if (bad & 0x80808080u) atomicOr(err, kErrBadBase64);
+  raise_bad(bad, err);
 }
 
 // Quads [q0, nq) one per thread: the tail after the fast kernel and unaligned buffers.
 // The final quad may carry padding, "xx==" (1 byte) or "xxx=" (2 bytes), and the bits
 // below its last character must be zero (std.base64: InvalidPadding otherwise).
 __global__ void __launch_bounds__(256) b64_decode_quads_kernel(const uint8_t* src, int64_t nq, int64_t q0,
-                                                               uint8_t* dst, int* err) {
+                                                               uint8_t* dst, int* err, int* pad) {
   uint32_t bad = 0;
   for (int64_t q = q0 + static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x; q < nq;
        q += static_cast<int64_t>(gridDim.x) * 256) {
@@ -169,6 +175,7 @@ __global__ void __launch_bounds__(256) b64_decode_quads_kernel(const uint8_t* sr
     uint32_t c2 = src[4 * q + 2], c3 = src[4 * q + 3];
     int p = 0;
     if (q == nq - 1 && c3 == '=') p = c2 == '=' ? 2 : 1;
+    if (q == nq - 1) __hip_atomic_store(pad, p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     if (p == 2) c2 = 'A';                // 'A' stands for the zero value of a padding position
     if (p >= 1) c3 = 'A';
     const uint32_t v = b64_group(b64_values4(c0 | (c1 << 8) | (c2 << 16) | (c3 << 24), bad));
@@ -178,7 +185,7 @@ __global__ void __launch_bounds__(256) b64_decode_quads_kernel(const uint8_t* sr
     if (p < 2) dst[3 * q + 1] = static_cast<uint8_t>(v >> 8);
     if (p < 1) dst[3 * q + 2] = static_cast<uint8_t>(v);
   }
-  if (bad & 0x80808080u) atomicOr(err, kErrBadBase64);
+  raise_bad(bad, err);
 }
 
 // ---- weights ------------------------------------------------------------------------------------
@@ -387,27 +394,22 @@ int pcp_base64_decode(pcp_ctx* ctx, const char* src, int64_t len, void* dst, int
   if (e != hipSuccess) return hip_fail(ctx, e, "hipSetDevice");
   if (len == 0) return PCP_OK;
   hipStream_t st = static_cast<hipStream_t>(stream);
-  char tail[2];
-  if ((e = hipMemcpyAsync(tail, src + len - 2, 2, hipMemcpyDeviceToHost, st)) != hipSuccess ||
-      (e = hipStreamSynchronize(st)) != hipSuccess)
-    return hip_fail(ctx, e, "reading the padding");
-  const int pad = tail[1] == '=' ? (tail[0] == '=' ? 2 : 1) : (tail[0] == '=' ? -1 : 0);
-  if (pad < 0) return fail(ctx, PCP_ERR_INVALID_ARG, "'=' before a non-padding character (InvalidPadding)");
   const int64_t nq = len / 4;
   const bool aligned = (reinterpret_cast<uintptr_t>(src) & 15u) == 0 && (reinterpret_cast<uintptr_t>(dst) & 3u) == 0;
   const int64_t nunits = aligned ? (nq - 1) / 4 : 0;   // the final quad (padding) always takes the byte path
   const bool timed = prof_begin(ctx, st);
   if (nunits > 0)
     b64_decode_kernel<<<static_cast<unsigned>((nunits + 256 * kUnits - 1) / (256 * kUnits)), 256, 0, st>>>(
-        reinterpret_cast<const u32x4*>(src), nunits, static_cast<uint32_t*>(dst), ctx->d_err);
+        reinterpret_cast<const u32x4*>(src), nunits, static_cast<uint32_t*>(dst), ctx->d_page->err);
   b64_decode_quads_kernel<<<grid_for(nq - 4 * nunits, 256), 256, 0, st>>>(
-      reinterpret_cast<const uint8_t*>(src), nq, 4 * nunits, static_cast<uint8_t*>(dst), ctx->d_err);
+      reinterpret_cast<const uint8_t*>(src), nq, 4 * nunits, static_cast<uint8_t*>(dst), ctx->d_page->err,
+      &ctx->d_page->b64_pad);
   prof_end(ctx, st, timed);
   if ((e = hipGetLastError()) != hipSuccess) return hip_fail(ctx, e, "base64 launch");
   if ((e = hipStreamSynchronize(st)) != hipSuccess) return hip_fail(ctx, e, "hipStreamSynchronize");
   const int rc = collect_device_errors(ctx);
   if (rc != PCP_OK) return rc;
-  *nbytes = nq * 3 - pad;
+  *nbytes = nq * 3 - ctx->page->b64_pad;
   return PCP_OK;
 }
 

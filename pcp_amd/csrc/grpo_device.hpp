@@ -21,13 +21,19 @@ constexpr float kLog2e = 1.44269504088896340736f;
 constexpr float kLn2 = 0.69314718055994530942f;
 constexpr float kNegInf = -__builtin_inff();
 
-// Device error bits, OR-ed into the context's flag word; the host maps them to
-// pcp_status codes after the stream is synchronised.
+// Device error conditions, raised in the context's host page (slot i for bit 1 << i); the
+// host maps them to pcp_status codes after the stream is synchronised.
 constexpr int kErrTokenRange = 1;
 constexpr int kErrNonFinite = 2;
 constexpr int kErrBadRagged = 4;   // rollout packing: offsets decrease or run past the token array
 constexpr int kErrBadBase64 = 8;   // base64: a character outside the alphabet or misplaced padding
 constexpr int kErrListedRow = 16;  // a row listed live by live_rows_kernel was not live in the row kernel
+
+// A store of 1 to the condition's own slot, not an atomic OR: the page is host memory, and
+// the link to the host carries no OR.
+__device__ __forceinline__ void raise_error(int* err, int bit) {
+  __hip_atomic_store(err + __builtin_ctz(static_cast<unsigned>(bit)), 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
 
 // v_exp_f32: 2^x. Used only for the per-element softmax terms, where results
 // below the fp32 normal range are irrelevant (they multiply a coefficient < 1).
@@ -332,7 +338,7 @@ struct RowArgs {
   float* logp;
   float* ref_logp;
   float* token_loss;
-  int* err;
+  int* err;                // the context's error slots (raise_error)
   int* next_row;           // persistent row kernel: rows handed out past the first grid
   // Without zero-fill: the live rows' indices and their count, filled by
   // live_rows_kernel before the persistent row kernel, which then visits only those
@@ -384,7 +390,7 @@ __device__ __forceinline__ RowMeta row_meta(const RowArgs& a, int64_t row) {
     const bool ignored = (r.id == PCP_IGNORE_INDEX);
     const bool in_range = (r.id >= 0) && (r.id < a.vocab);
     if (r.w != 0.f && !ignored && !in_range) {
-      if (threadIdx.x == 0) atomicOr(a.err, kErrTokenRange);
+      if (threadIdx.x == 0) raise_error(a.err, kErrTokenRange);
     }
     r.live = (r.w != 0.f) && in_range;
   }

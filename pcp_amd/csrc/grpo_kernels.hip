@@ -56,7 +56,7 @@ __device__ __forceinline__ void zero_row_scalar(void* dl, int64_t row_elem, int6
 
 __device__ __forceinline__ void flag_nonfinite(const RowArgs& a, float lse, float lr_lse) {
   if (threadIdx.x == 0 && !(__builtin_isfinite(lse) && __builtin_isfinite(lr_lse)))
-    atomicOr(a.err, kErrNonFinite);
+    raise_error(a.err, kErrNonFinite);
 }
 
 // A row that may start off 16 bytes: its 16-byte-aligned interior of nv vectors, and
@@ -209,7 +209,7 @@ __device__ __forceinline__ int64_t resident_row(const RowArgs& a, const int64_t 
       // inputs changed under the launch. Fail loudly (PCP_ERR_INVALID_ARG); this
       // workgroup's claimed rows stay unprocessed. (Loading the next row here as well
       // as in the live path's dlogits pass made hipcc spill 75-110 VGPRs.)
-      if (tid == 0) atomicOr(a.err, kErrListedRow);
+      if (tid == 0) raise_error(a.err, kErrListedRow);
     }
     return -1;
   }
@@ -564,7 +564,7 @@ __global__ void __launch_bounds__(256) live_rows_kernel(RowArgs a) {
       if (a.mask) w = a.mask_u8 ? (static_cast<const uint8_t*>(a.mask)[tix] ? 1.f : 0.f)
                                 : static_cast<const float*>(a.mask)[tix];
       const bool in_range = id >= 0 && id < a.vocab;
-      if (w != 0.f && id != PCP_IGNORE_INDEX && !in_range) atomicOr(a.err, kErrTokenRange);
+      if (w != 0.f && id != PCP_IGNORE_INDEX && !in_range) raise_error(a.err, kErrTokenRange);
       live = w != 0.f && in_range;
       if (!live) {
         if (a.logp) a.logp[tix] = 0.f;

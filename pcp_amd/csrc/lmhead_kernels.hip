@@ -1170,7 +1170,7 @@ __global__ void __launch_bounds__(256) lm_terms_kernel(RowArgs ra, LmTermsArgs a
     else if (ra.mask_u8) r.w = static_cast<const uint8_t*>(ra.mask)[r.tix] ? 1.f : 0.f;
     else r.w = static_cast<const float*>(ra.mask)[r.tix];
     const bool in_range = r.id >= 0 && r.id < ra.vocab;
-    if (r.w != 0.f && r.id != PCP_IGNORE_INDEX && !in_range) atomicOr(ra.err, kErrTokenRange);
+    if (r.w != 0.f && r.id != PCP_IGNORE_INDEX && !in_range) raise_error(ra.err, kErrTokenRange);
     r.live = r.tok && r.w != 0.f && in_range;
   }
   float lp = 0.f, lr = 0.f;
@@ -1181,7 +1181,7 @@ __global__ void __launch_bounds__(256) lm_terms_kernel(RowArgs ra, LmTermsArgs a
     // Non-finite logits of a live token poison its log-sum-exp (NaN propagates
     // through the partial merges); flag it like the logits-input path does.
     const float l2 = a.lse2[c], rl2 = a.ref_tgt ? a.ref_lse2[c] : 0.f;
-    if (!(__builtin_isfinite(l2) && __builtin_isfinite(rl2))) atomicOr(ra.err, kErrNonFinite);
+    if (!(__builtin_isfinite(l2) && __builtin_isfinite(rl2))) raise_error(ra.err, kErrNonFinite);
     lp = a.tgt[c] - l2 * kLn2;
     lr = a.ref_tgt ? a.ref_tgt[c] - rl2 * kLn2 : 0.f;
     tt = token_terms(ra, r, lp, lr);

@@ -348,7 +348,7 @@ int run_lm(pcp_ctx* ctx, const pcp_lmhead_args* a) {
   ra.logp = a->logp;
   ra.ref_logp = a->ref_logp;
   ra.token_loss = tl;
-  ra.err = ctx->d_err;
+  ra.err = ctx->d_page->err;
   ra.vocab = V;
   ra.rows = T;
   ra.logit_stride = T;

@@ -69,7 +69,7 @@ __global__ void __launch_bounds__(256) pack_kernel(PackArgs a) {
     lc = a.co[r + 1] - c0;
     const bool ok = p0 >= 0 && lp >= 0 && p0 + lp <= a.npt && c0 >= 0 && lc >= 0 && c0 + lc <= a.nct;
     if (!ok) {
-      if (threadIdx.x == 0) atomicOr(a.err, kErrBadRagged);
+      if (threadIdx.x == 0) raise_error(a.err, kErrBadRagged);
       lp = 0;
       lc = 0;
     }
@@ -100,6 +100,8 @@ struct StatsPart {
   int64_t nan_count;
   int64_t inf_count;
 };
+
+static_assert(sizeof(StatsPart) <= sizeof(HostPage::stats), "the page holds one result");
 
 // Several tensors in one launch: tensor t's chunks of kStatsChunk elements are chunks
 // [first[t], first[t + 1]) of the launch. The table travels in the kernel's arguments
@@ -389,7 +391,7 @@ int pcp_pack_rollouts(pcp_ctx* ctx, const int64_t* prompt_tokens, int64_t n_prom
   if (e != hipSuccess) return hip_fail(ctx, e, "hipSetDevice");
   hipStream_t st = static_cast<hipStream_t>(stream);
   PackArgs a{prompt_tokens, prompt_offsets, completion_tokens, completion_offsets, n_prompt_tokens,
-             n_completion_tokens, n_rollouts, seq_len, ids, mask, ctx->d_err};
+             n_completion_tokens, n_rollouts, seq_len, ids, mask, ctx->d_page->err};
   pack_kernel<<<dim3(static_cast<unsigned>(n_rows)), dim3(256), 0, st>>>(a);
   if ((e = hipGetLastError()) != hipSuccess) return hip_fail(ctx, e, "pack launch");
   return finish(ctx, st);
@@ -421,7 +423,7 @@ int pcp_grad_stats_compute_many(pcp_ctx* ctx, int n_tensors, const float* const*
     // A launch takes up to kStatsTensors tensors and writes at most kStatsBlocks partials.
     const int64_t launches = (n_tensors + kStatsTensors - 1) / kStatsTensors;
     const int64_t cap = chunks < launches * kStatsBlocks ? chunks : launches * kStatsBlocks;
-    int rc = ensure_scratch(ctx, sizeof(StatsPart) * static_cast<size_t>(cap + 1));
+    int rc = ensure_scratch(ctx, sizeof(StatsPart) * static_cast<size_t>(cap));
     if (rc != PCP_OK) return rc;
     StatsPart* parts = static_cast<StatsPart*>(ctx->scratch);
     int nparts = 0;
@@ -441,11 +443,10 @@ int pcp_grad_stats_compute_many(pcp_ctx* ctx, int n_tensors, const float* const*
       stats_kernel<<<grid, 256, 0, st>>>(b, parts + nparts);
       nparts += grid;
     }
-    stats_final_kernel<<<1, 1024, 0, st>>>(parts, nparts, parts + cap);
+    stats_final_kernel<<<1, 1024, 0, st>>>(parts, nparts, reinterpret_cast<StatsPart*>(ctx->d_page->stats));
     if ((e = hipGetLastError()) != hipSuccess) return hip_fail(ctx, e, "statistics launch");
-    if ((e = hipMemcpyAsync(&h, parts + cap, sizeof(h), hipMemcpyDeviceToHost, st)) != hipSuccess)
-      return hip_fail(ctx, e, "reading statistics");
     if ((e = hipStreamSynchronize(st)) != hipSuccess) return hip_fail(ctx, e, "hipStreamSynchronize");
+    std::memcpy(&h, ctx->page->stats, sizeof(h));
   }
   if (!accumulate) *stats = pcp_grad_stats{0.0, 0.0, 0.f, 0, 0, 0};
   stats->sumsq += h.sumsq;
