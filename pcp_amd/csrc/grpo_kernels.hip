@@ -466,7 +466,7 @@ __device__ __forceinline__ int64_t resident_row(const RowArgs& a, const int64_t 
 // by live_rows_kernel (a separate instance, so the zero-fill loop is compiled as before).
 template <typename TI, typename TO, int BLOCK, int NCH, int RB, bool EDGE, bool CACHE, bool LIST>
 __global__ void __launch_bounds__(BLOCK) grpo_resident_kernel(RowArgs a) {
-  __shared__ float lds[4 * (BLOCK / 64)];
+  __shared__ __align__(16) float lds[4 * (BLOCK / 64)];
   __shared__ int s_next[2];
   if constexpr (LIST) {
     // Without zero-fill: live_rows_kernel listed the live rows and counted them earlier
@@ -622,7 +622,7 @@ template <typename TI, int BLOCK, int U, bool REF>
 __global__ void __launch_bounds__(BLOCK) grpo_fwd_kernel(RowArgs a) {
   constexpr int EPV = 16 / TI::kBytes;
   constexpr uint32_t kStep = BLOCK * 16u;   // bytes between a lane's vectors in one batch
-  __shared__ float lds[4 * (BLOCK / 64)];
+  __shared__ __align__(16) float lds[4 * (BLOCK / 64)];
   const int tid = threadIdx.x;
   const int64_t row = blockIdx.x;
   const RowMeta r = row_meta(a, row);
@@ -737,7 +737,7 @@ template <typename TI, typename TO, int BLOCK, int U, bool VEC, bool NT1>
 __global__ void __launch_bounds__(BLOCK) grpo_stream_kernel(RowArgs a) {
   using IO = StreamIO<TI, VEC>;
   constexpr int EPV = IO::EPV;
-  __shared__ float lds[4 * (BLOCK / 64)];
+  __shared__ __align__(16) float lds[4 * (BLOCK / 64)];
   const int tid = threadIdx.x;
   const int64_t row = blockIdx.x;
   const RowMeta r = row_meta(a, row);
