@@ -462,12 +462,32 @@ __device__ __forceinline__ int64_t resident_row(const RowArgs& a, const int64_t 
 // step i, while slot (i - 1) & 1 may still be read; the barrier at the end of step i
 // orders the reads of slot i & 1 before its next write, in step i + 2.
 
+// Rows of up to 32 KB (256 lanes, up to 8 chunks) are dealt in grid strides instead: the
+// counter is one address, whose atomics complete at about 85 a microsecond on this chip,
+// and such rows go by faster than that. Clip-KL, dead rows zero-filled, ms before and
+// after: 131,072 rows of 1000 bf16 1.53 -> .426, 4096 bf16 1.20 -> .417, configuration 1's
+// 1024 rows of 1024 f32 43.5 -> 32 us (all of it the counter: no row is left to claim
+// there, and a launch whose first grid covers its rows now leaves the counter alone).
+// Wider rows keep the counter, which balances live against dead rows: dealt in strides,
+// 8192 rows of 16,000 f32 took 229 us against 201, of 50,257 bf16 426 against 356.
+template <int BLOCK, int NCH>
+constexpr bool kResStatic = BLOCK * NCH <= 2048;
+
 // LIST: the instance for launches without zero-fill, which visit the live rows listed
 // by live_rows_kernel (a separate instance, so the zero-fill loop is compiled as before).
 template <typename TI, typename TO, int BLOCK, int NCH, int RB, bool EDGE, bool CACHE, bool LIST>
 __global__ void __launch_bounds__(BLOCK) grpo_resident_kernel(RowArgs a) {
+  // Rows past the first grid: claimed from the launch's counter, or, for narrow rows
+  // (kResStatic), dealt in grid strides.
+  constexpr bool kStatic = kResStatic<BLOCK, NCH>;
   __shared__ __align__(16) float lds[4 * (BLOCK / 64)];
   __shared__ int s_next[2];
+  // Thread 0's claim for step i + 1 of a launch of n rows (no counter when the first grid
+  // covers them all).
+  auto next_claim = [&](int i, int64_t n) {
+    if (kStatic || threadIdx.x != 0) return;
+    s_next[i & 1] = n > static_cast<int64_t>(gridDim.x) ? atomicAdd(a.next_row, 1) + static_cast<int>(gridDim.x) : INT32_MAX;
+  };
   if constexpr (LIST) {
     // Without zero-fill: live_rows_kernel listed the live rows and counted them earlier
     // on the stream. When fewer than half the rows are live the launch visits the listed
@@ -499,9 +519,9 @@ __global__ void __launch_bounds__(BLOCK) grpo_resident_kernel(RowArgs a) {
         }
         int claim = idx + static_cast<int>(gridDim.x);
         for (;;) {
-          int listed = -1, taken = 0;
+          int listed = -1, taken = claim - static_cast<int>(gridDim.x);
           if (threadIdx.x == 0) {
-            taken = atomicAdd(a.next_row, 1);
+            if (!kStatic && claim < n) taken = atomicAdd(a.next_row, 1);
             listed = a.row_list[min(claim, n - 1)];
           }
           row = resident_row<TI, TO, BLOCK, NCH, RB, false, CACHE, true>(a, row, lds, xv, listed, claim < n, s_next);
@@ -512,11 +532,11 @@ __global__ void __launch_bounds__(BLOCK) grpo_resident_kernel(RowArgs a) {
       } else {
         int64_t idx = blockIdx.x;
         for (int i = 0; idx < n; ++i) {
-          if (threadIdx.x == 0) s_next[i & 1] = atomicAdd(a.next_row, 1) + static_cast<int>(gridDim.x);
+          next_claim(i, n);
           u32x4 xv[NCH];
           resident_row<TI, TO, BLOCK, NCH, RB, EDGE, CACHE>(a, a.row_list[idx], lds, xv);
           __syncthreads();   // s_next visible; this row's LDS reads done before the next row writes
-          idx = s_next[i & 1];
+          idx = kStatic ? idx + gridDim.x : s_next[i & 1];
         }
         return;
       }
@@ -532,11 +552,11 @@ __global__ void __launch_bounds__(BLOCK) grpo_resident_kernel(RowArgs a) {
     constexpr int kSP = LIST ? kBufNT : kBufNTSystem;
     int64_t row = blockIdx.x;
     for (int i = 0; row < a.nrows; ++i) {
-      if (threadIdx.x == 0) s_next[i & 1] = atomicAdd(a.next_row, 1) + static_cast<int>(gridDim.x);
+      next_claim(i, a.nrows);
       u32x4 xv[NCH];
       resident_row<TI, TO, BLOCK, NCH, RB, EDGE, CACHE, false, kSP>(a, row, lds, xv);
       __syncthreads();   // s_next visible; this row's LDS reads done before the next row writes
-      row = s_next[i & 1];
+      row = kStatic ? row + gridDim.x : s_next[i & 1];
     }
   }
 }
@@ -1182,10 +1202,16 @@ hipError_t launch_fwd(const RowArgs& a, int64_t nrows, hipStream_t st) {
 struct ResCfg {
   int block, nch;
 };
+// (256, 8) holds rows of up to 32 KB: several workgroups share a CU, so one row's loads run
+// under the others' merges and stores. Against (1024, 2) there, 8192 rows of 8000 f32 145
+// -> 131 us, 25,728 of 16,000 bf16 468 -> 349 us (part of it kResStatic). For wider rows more
+// lanes are better: 512 lanes of 8, 13 and 16 chunks measured 322 against 332 us for 32,000
+// bf16 but 211 against 201 for 16,000 f32, 379 against 355 for 50,257 bf16 and 412 against 375 for
+// 65,000; 256 lanes of 16, 25 and 32 chunks were slower still.
 // (1024, 24) would spill at the 128-VGPR budget of a 1024-lane workgroup, so rows
 // wider than 20480 16-byte vectors (V > 163840 for 16-bit logits) stream instead.
-constexpr ResCfg kResCfgs[] = {{256, 1},   {256, 2},   {256, 4},   {1024, 2}, {1024, 4},
-                               {1024, 8},  {1024, 12}, {1024, 16}, {1024, 19}, {1024, 20}};
+constexpr ResCfg kResCfgs[] = {{256, 1},  {256, 2},   {256, 4},   {256, 8},   {1024, 4},
+                               {1024, 8}, {1024, 12}, {1024, 16}, {1024, 19}, {1024, 20}};
 
 // Rows off 16 bytes (EDGE) need dlogits of the logits' element type. Only bf16 -> bf16
 // rows have the f16 softmax cache, so only they have instances without it (exact).
@@ -1210,7 +1236,7 @@ hipError_t dispatch_resident(int cfg, bool edge, bool exact, const RowArgs& a, i
     case 0: return launch_resident_cfg<TI, TO, 256, 1>(edge, exact, a, nrows, st);
     case 1: return launch_resident_cfg<TI, TO, 256, 2>(edge, exact, a, nrows, st);
     case 2: return launch_resident_cfg<TI, TO, 256, 4>(edge, exact, a, nrows, st);
-    case 3: return launch_resident_cfg<TI, TO, 1024, 2>(edge, exact, a, nrows, st);
+    case 3: return launch_resident_cfg<TI, TO, 256, 8>(edge, exact, a, nrows, st);
     case 4: return launch_resident_cfg<TI, TO, 1024, 4>(edge, exact, a, nrows, st);
     case 5: return launch_resident_cfg<TI, TO, 1024, 8>(edge, exact, a, nrows, st);
     case 6: return launch_resident_cfg<TI, TO, 1024, 12>(edge, exact, a, nrows, st);

@@ -255,3 +255,32 @@ def test_no_zero_fill_live_counts(count_inputs, n_live, dt):
     assert bool((want.dlogits[~live] == 0).all())
     for f in ("loss", "logp", "ref_logp", "token_loss", "advantages"):
         assert torch.equal(getattr(got, f), getattr(want, f)), f
+
+
+@pytest.mark.parametrize("zero_fill, longest", [(True, 128), (False, 128), (False, 40)])
+@pytest.mark.parametrize("dtype, V", [("bf16", 64), ("bf16", 1001), ("bf16", 16384), ("bf16", 16392), ("f32", 8192),
+                                      ("f32", 1030), ("f16", 8200)])
+def test_rows_past_the_first_grid(dtype, V, zero_fill, longest):
+    """Narrow rows (256 lanes x 1 to 8 chunks, aligned and not) are dealt in grid strides, wider
+    ones from the counter. A row's outputs depend on its own data only, so the last 4 of 72
+    sequences (9,216 rows, more than two grids of the widest launch) must come out bit for bit
+    as in a call of their own (512 rows: one grid). longest 40 lists under half of the rows."""
+    dt = {"bf16": torch.bfloat16, "f16": torch.float16, "f32": torch.float32}[dtype]
+    S, T = 72, 128
+    gen = torch.Generator(device="cuda").manual_seed(V)
+    x = (torch.randn((S, T, V), generator=gen, device="cuda") * 3).to(dt)
+    r = (x.float() + 0.1 * torch.randn((S, T, V), generator=gen, device="cuda")).to(dt)
+    ids = torch.randint(0, V, (S, T), generator=gen, device="cuda")
+    lengths = torch.randint(1, longest + 1, (S, 1), generator=gen, device="cuda")
+    mask = (torch.arange(T, device="cuda")[None] < lengths).float()
+    adv = torch.randn(S, generator=gen, device="cuda")
+    old = -torch.rand((S, T), generator=gen, device="cuda") * 9
+
+    def call(sl):
+        out = grpo.grpo_loss_fwd_bwd(x[sl], ids[sl], mask[sl], advantages=adv[sl], ref_logits=r[sl], old_logp=old[sl],
+                                     loss_mode=LossMode.GRPO_CLIP_KL, loss_norm=float(S), zero_fill=zero_fill,
+                                     dlogits=torch.full_like(x[sl], 7.0))
+        return out.dlogits, out.logp, out.ref_logp, out.token_loss
+
+    for whole, own in zip(call(slice(0, S)), call(slice(S - 4, S))):
+        assert torch.equal(whole[S - 4:], own)
