@@ -110,6 +110,10 @@ int collect_device_errors(pcp_ctx* ctx);
 // through the error word).
 int add_pending(pcp_ctx* ctx, hipStream_t st);
 
+// pcp_grpo_loss_fwd_bwd with the row kernel planned for a call of plan_nrows rows, of
+// which this one is a group.
+int loss_fwd_bwd_planned(pcp_ctx* ctx, const pcp_grpo_args* a, int64_t plan_nrows);
+
 // pcp_profile_start/stop: HIP events around a timed launch on its stream. prof_begin
 // returns whether this launch is timed (profiling on and an event pair left).
 inline bool prof_begin(pcp_ctx* ctx, hipStream_t st) {

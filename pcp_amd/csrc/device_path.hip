@@ -195,7 +195,8 @@ int finish(pcp_ctx* ctx, const pcp_grpo_args* a, hipStream_t st) {
 
 // noalloc: take the work buffers from the device's static scratch array instead of
 // the context's grow-only buffer (no allocation of any kind on this path).
-int run(pcp_ctx* ctx, const pcp_grpo_args* a, Op op, bool noalloc = false) {
+// plan_nrows: rows to plan for (0: the call's own).
+int run(pcp_ctx* ctx, const pcp_grpo_args* a, Op op, bool noalloc = false, int64_t plan_nrows = 0) {
   Geo g;
   int rc = validate(a, op, &g);
   if (rc != PCP_OK) {
@@ -203,14 +204,33 @@ int run(pcp_ctx* ctx, const pcp_grpo_args* a, Op op, bool noalloc = false) {
     return rc;
   }
 
+  // The row kernel's plan.
+  const void* ref = op == kLogprob || a->loss_mode == PCP_LOSS_GRPO_CLIP_KL ? a->ref_logits : nullptr;
+  void* dl = op == kLoss ? a->dlogits : nullptr;
+  const bool al = aligned16(a->logits) && (!ref || aligned16(ref)) && (!dl || aligned16(dl));
+  const bool edge_ok = !dl || (a->dlogits_dtype == a->logits_dtype && ((reinterpret_cast<uintptr_t>(a->logits) ^
+                                                                         reinterpret_cast<uintptr_t>(dl)) & 15u) == 0);
+  auto plan_for = [&](int64_t rows) {
+    RowPlan p = plan_rows(dtype_bytes(a->logits_dtype), g.vocab, al, edge_ok, dl == nullptr,
+                          (a->flags & PCP_FLAG_FORCE_STREAMING) != 0, rows);
+    p.exact = (a->flags & PCP_FLAG_EXACT_BF16) ? 1 : 0;
+    return p;
+  };
+  RowPlan plan = plan_for(plan_nrows ? plan_nrows : g.nrows);
+
   // Scratch: adv | seq_len | seq_scale | seq_val | loss | row counter, live-row count,
-  // loss ticket | token_loss | live-row list (without zero-fill).
+  // loss ticket | token_loss | live-row list (without zero-fill) | row parts.
   const size_t sv = round256(sizeof(float) * g.n_seq);
   const bool need_tl = (op == kLoss) && a->token_loss == nullptr;
   const size_t tl_bytes = need_tl ? round256(sizeof(float) * g.n_seq * g.tstride) : 0;
   const bool need_list = (op == kLoss) && a->dlogits != nullptr && (a->flags & PCP_FLAG_NO_ZERO_FILL);
   const size_t list_bytes = need_list ? round256(sizeof(int) * static_cast<size_t>(g.nrows)) : 0;
-  const size_t need = 4 * sv + 512 + tl_bytes + list_bytes;
+  size_t part_bytes = round256(plan_part_bytes(plan, g.nrows));
+  if (noalloc && 4 * sv + 512 + tl_bytes + list_bytes + part_bytes > PCP_NOALLOC_SCRATCH_BYTES) {
+    plan = plan_for(INT64_MAX);   // no room for the parts' results: a row per workgroup
+    part_bytes = 0;
+  }
+  const size_t need = 4 * sv + 512 + tl_bytes + list_bytes + part_bytes;
   if (noalloc && need > PCP_NOALLOC_SCRATCH_BYTES)
     return fail(ctx, PCP_ERR_OVERFLOW,
                 "the allocation-free call needs %zu bytes of work space, more than its %u-byte array: pass "
@@ -242,6 +262,7 @@ int run(pcp_ctx* ctx, const pcp_grpo_args* a, Op op, bool noalloc = false) {
 
   RowArgs ra;
   std::memset(&ra, 0, sizeof(ra));
+  if (part_bytes) ra.part = reinterpret_cast<float4*>(sp + 4 * sv + 512 + tl_bytes + list_bytes);
   ra.logits = a->logits;
   ra.ids = a->ids;
   ra.mask = a->mask;
@@ -261,12 +282,14 @@ int run(pcp_ctx* ctx, const pcp_grpo_args* a, Op op, bool noalloc = false) {
   ra.logp = a->logp;
   ra.ref_logp = a->ref_logp;
 
+  // With the row in parts its first kernel does the prep.
+  const bool prep_in_rows = op == kLoss && plan.kind == RowPlan::kParts && g.nrows + g.n_seq <= 65535;
+  StepPrepArgs pa;
+  std::memset(&pa, 0, sizeof(pa));
   if (op == kLoss) {
     // One launch: advantages (or the copy of the given ones), per-sequence lengths, and
     // the row kernel's and the loss ticket's counters zeroed.
     const float* adv = a->advantages ? a->advantages : s_adv;
-    StepPrepArgs pa;
-    std::memset(&pa, 0, sizeof(pa));
     pa.mask = a->mask;
     pa.mask_u8 = ra.mask_u8;
     pa.n_seq = g.n_seq;
@@ -285,10 +308,9 @@ int run(pcp_ctx* ctx, const pcp_grpo_args* a, Op op, bool noalloc = false) {
     pa.zero[0] = s_next;
     pa.zero[1] = s_list ? s_count : nullptr;
     pa.zero[2] = s_done;
-    e = launch_step_prep(pa, st);
-    if (e != hipSuccess) return hip_fail(ctx, e, "step prep launch");
+    if (!prep_in_rows && (e = launch_step_prep(pa, st)) != hipSuccess) return hip_fail(ctx, e, "step prep launch");
     ra.counters_zeroed = 1;
-    ra.ref_logits = (a->loss_mode == PCP_LOSS_GRPO_CLIP_KL) ? a->ref_logits : nullptr;
+    ra.ref_logits = ref;
     ra.old_logp = a->old_logp;
     ra.adv = adv;
     ra.seq_scale = s_scale;
@@ -298,25 +320,17 @@ int run(pcp_ctx* ctx, const pcp_grpo_args* a, Op op, bool noalloc = false) {
     ra.clip_eps = a->clip_eps;
     ra.kl_beta = a->kl_beta;
   } else {
-    ra.ref_logits = a->ref_logits;
+    ra.ref_logits = ref;
   }
 
-  const int in_bytes = dtype_bytes(a->logits_dtype);
-  const bool al = aligned16(a->logits) && (!ra.ref_logits || aligned16(ra.ref_logits)) &&
-                  (!ra.dlogits || aligned16(ra.dlogits));
-  const bool edge_ok = !ra.dlogits || (a->dlogits_dtype == a->logits_dtype &&
-                                       ((reinterpret_cast<uintptr_t>(a->logits) ^
-                                         reinterpret_cast<uintptr_t>(ra.dlogits)) & 15u) == 0);
-  RowPlan plan = plan_rows(in_bytes, g.vocab, al, edge_ok, ra.dlogits == nullptr,
-                           (a->flags & PCP_FLAG_FORCE_STREAMING) != 0);
-  plan.exact = (a->flags & PCP_FLAG_EXACT_BF16) ? 1 : 0;
   const int out_dt = ra.dlogits ? a->dlogits_dtype : a->logits_dtype;
   const bool timed = ctx->prof_on && ctx->prof_used < static_cast<int>(ctx->prof_start.size());
   if (timed) {
     e = hipEventRecord(ctx->prof_start[ctx->prof_used], st);
     if (e != hipSuccess) return hip_fail(ctx, e, "hipEventRecord");
   }
-  e = launch_rows(plan, a->logits_dtype, out_dt == PCP_F32 ? PCP_F32 : a->logits_dtype, ra, g.nrows, st);
+  e = launch_rows(plan, a->logits_dtype, out_dt == PCP_F32 ? PCP_F32 : a->logits_dtype, ra,
+                  prep_in_rows ? &pa : nullptr, g.nrows, st);
   if (e != hipSuccess) return hip_fail(ctx, e, "row kernel launch");
   if (timed) {
     e = hipEventRecord(ctx->prof_stop[ctx->prof_used++], st);
@@ -333,6 +347,11 @@ int run(pcp_ctx* ctx, const pcp_grpo_args* a, Op op, bool noalloc = false) {
 }
 
 }  // namespace
+
+int loss_fwd_bwd_planned(pcp_ctx* ctx, const pcp_grpo_args* a, int64_t plan_nrows) {
+  return run(ctx, a, kLoss, false, plan_nrows);
+}
+
 }  // namespace pcp
 
 using namespace pcp;

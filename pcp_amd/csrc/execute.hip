@@ -280,7 +280,7 @@ int run_loss_groups(pcp_ctx* ctx, const pcp_grpo_args& full, const In& L, const 
     g.loss_norm = gtot;
     g.flags = PCP_FLAG_ASYNC;
     g.stream = run;
-    if ((rc = pcp_grpo_loss_fwd_bwd(ctx, &g)) != PCP_OK) return rc;
+    if ((rc = loss_fwd_bwd_planned(ctx, &g, S * T)) != PCP_OK) return rc;
     e = drain.mark(run, down);
     if (e == hipSuccess)
       e = hipMemcpyAsync(static_cast<char*>(host_dl) + off, static_cast<char*>(full.dlogits) + off, len,

@@ -268,8 +268,15 @@ __device__ __forceinline__ float ms_rescale(float s, float m, float nm) {
   return (s == 0.f) ? 0.f : s * hw_exp2(m - ms_ref(nm));
 }
 
-// log-sum-exp (natural units) of a merged state.
-__device__ __forceinline__ float ms_lse(float m, float s) { return (m + log2f(s)) * kLn2; }
+// log-sum-exp (natural units) of a merged state, to a few 1e-8: m and the exponent of s
+// add up exactly in f64, and log2f of s's mantissa is within an ulp of 1. In f32 the sum
+// m + log2f(s) and its product round at the size of the log-sum-exp (16 at V = 151,936:
+// 1e-6 of every log-prob, ratio and KL term).
+__device__ __forceinline__ double ms_lse(float m, float s) {
+  const int k = __builtin_amdgcn_frexp_expf(s);
+  const float f = log2f(__builtin_amdgcn_frexp_mantf(s));
+  return (static_cast<double>(m) + static_cast<double>(k) + static_cast<double>(f)) * 0.69314718055994530942;
+}
 
 // v of the lane that DPP control CTRL names, `id` where there is none (or ROWS masks this
 // lane's 16-lane row off).
@@ -381,6 +388,7 @@ struct RowArgs {
   // rows. nullptr: every row in order.
   int* row_list;
   int* row_count;
+  float4* part;            // RowPlan::kParts: [nrows, parts] (policy m, s, reference m, s)
   int64_t nrows;           // logits rows of the launch
   int64_t vocab;
   int64_t rows;
@@ -458,8 +466,9 @@ struct TokenTerms {
   float coef;  // c = d loss / d logp (already includes m / (loss_norm * L_s))
 };
 
-__device__ __forceinline__ TokenTerms token_terms(const RowArgs& a, const RowMeta& r, float lp,
-                                                  float lr) {
+// lp, lr: log-probs in f64, so that the differences below lose nothing of them.
+__device__ __forceinline__ TokenTerms token_terms(const RowArgs& a, const RowMeta& r, double lp,
+                                                  double lr) {
   TokenTerms o;
   if (a.adv == nullptr) {  // forward-only request: no loss terms
     o.loss = 0.f;
@@ -470,15 +479,14 @@ __device__ __forceinline__ TokenTerms token_terms(const RowArgs& a, const RowMet
   const float scale = a.seq_scale[r.seq] * r.w;
   if (a.loss_mode == PCP_LOSS_REINFORCE) {
     // token_losses = -logp * mask; seq_nll * adv; mean  (export_qwen_forward.py:156-163)
-    o.loss = r.w * (-lp);
+    o.loss = r.w * static_cast<float>(-lp);
     o.coef = -A * scale;
   } else {
-    const float old = a.old_logp ? a.old_logp[r.tix] : lp;
-    const float rho = expf(lp - old);
+    const float rho = a.old_logp ? expf(static_cast<float>(lp - static_cast<double>(a.old_logp[r.tix]))) : 1.f;
     const float lo = 1.f - a.clip_eps, hi = 1.f + a.clip_eps;
     const float rc = fminf(fmaxf(rho, lo), hi);
     const float surr = fminf(rho * A, rc * A);
-    const float dlr = lr - lp;
+    const float dlr = static_cast<float>(lr - lp);
     o.loss = r.w * (-surr + a.kl_beta * kl_k3(dlr));
     // The min picks the unclipped branch (gradient -A*rho) unless the ratio left the
     // trust region on the side the advantage's sign rewards.

@@ -27,6 +27,7 @@
 #include <stdint.h>
 
 #include <atomic>
+#include <cstring>
 
 #include "grpo_device.hpp"
 #include "grpo_launch.hpp"
@@ -54,7 +55,7 @@ __device__ __forceinline__ void zero_row_scalar(void* dl, int64_t row_elem, int6
   for (int64_t i = threadIdx.x; i < v; i += BLOCK) store1<TO>(dl, row_elem + i, 0.f);
 }
 
-__device__ __forceinline__ void flag_nonfinite(const RowArgs& a, float lse, float lr_lse) {
+__device__ __forceinline__ void flag_nonfinite(const RowArgs& a, double lse, double lr_lse) {
   if (threadIdx.x == 0 && !(__builtin_isfinite(lse) && __builtin_isfinite(lr_lse)))
     raise_error(a.err, kErrNonFinite);
 }
@@ -376,15 +377,15 @@ __device__ __forceinline__ int64_t resident_row(const RowArgs& a, const int64_t 
   }
   block_merge2<BLOCK>(pm, ps, rm, rs, lds);
   const float lse2 = pm + log2f(ps);
-  const float lse = lse2 * kLn2;
-  const float rlse = has_ref ? ms_lse(rm, rs) : 0.f;
+  const double lse = ms_lse(pm, ps);
+  const double rlse = has_ref ? ms_lse(rm, rs) : 0.;
   flag_nonfinite(a, lse, rlse);
 
   // 4. Token math.
-  const float lp = xy - lse;
-  const float lr = ry - rlse;
+  const double lp = xy - lse;
+  const double lr = ry - rlse;
   const TokenTerms tt = token_terms(a, r, lp, lr);
-  write_token_outputs(a, r, lp, lr, tt.loss);
+  write_token_outputs(a, r, static_cast<float>(lp), static_cast<float>(lr), tt.loss);
   if constexpr (!PF) {   // PF launches always write dlogits
     if (a.dlogits == nullptr) return -1;   // forward only (log-probs)
   }
@@ -714,14 +715,326 @@ __global__ void __launch_bounds__(BLOCK) grpo_fwd_kernel(RowArgs a) {
   }
 
   block_merge2<BLOCK>(pm, ps, rm, rs, lds);
-  const float lse2 = pm + log2f(ps);
-  const float lse = lse2 * kLn2;
-  const float rlse = REF ? ms_lse(rm, rs) : 0.f;
+  const double lse = ms_lse(pm, ps);
+  const double rlse = REF ? ms_lse(rm, rs) : 0.;
   flag_nonfinite(a, lse, rlse);
-  const float lp = xy - lse;
-  const float lr = ry - rlse;
+  const double lp = xy - lse;
+  const double lr = ry - rlse;
   const TokenTerms tt = token_terms(a, r, lp, lr);
-  write_token_outputs(a, r, lp, lr, tt.loss);
+  write_token_outputs(a, r, static_cast<float>(lp), static_cast<float>(lr), tt.loss);
+}
+
+// ---------------------------------------------------------------------------
+// Sequence lengths and advantages: the work before the row kernel.
+// ---------------------------------------------------------------------------
+
+// Deterministic workgroup sum: fixed per-lane order, xor butterfly (commutative,
+// so every lane agrees), fixed cross-wave order. Result on every thread.
+template <int BLOCK>
+__device__ __forceinline__ float block_sum(float v, float* lds) {
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off);
+  constexpr int NW = BLOCK / 64;
+  if constexpr (NW > 1) {
+    if ((threadIdx.x & 63) == 0) lds[threadIdx.x >> 6] = v;
+    __syncthreads();
+    v = lds[0];
+#pragma unroll
+    for (int w = 1; w < NW; ++w) v += lds[w];
+    __syncthreads();
+  }
+  return v;
+}
+
+constexpr int kSmallBlock = 256;
+
+// Group-relative advantages, restating rl_shepherd.zig:466-478 operation by
+// operation in IEEE fp32: sequential sum, mean = sum / n, sequential sum of
+// (r-mean)*(r-mean), std = sqrt(ssd / n) + eps, (r-mean)/std. hipcc contracts
+// a*b+c into an FMA by default (also inside the __fmul_rn/__fadd_rn helpers,
+// which are compiled outside this scope), so the arithmetic is written with
+// plain operators under contract(off); fp32 '/' and sqrtf are correctly rounded
+// (hipcc's default -fhip-fp32-correctly-rounded-divide-sqrt).
+// The group of rewards [i, e): adv[k] (and adv2[k] when adv2 is not null).
+__device__ __forceinline__ void group_advantages(const float* r, int64_t i, int64_t e, float eps, float* adv,
+                                                 float* adv2) {
+#pragma clang fp contract(off)
+  const float cnt = static_cast<float>(e - i);
+  float sum = 0.f;
+  for (int64_t k = i; k < e; ++k) sum = sum + r[k];
+  const float mean = sum / cnt;
+  float ssd = 0.f;
+  for (int64_t k = i; k < e; ++k) {
+    const float d = r[k] - mean;
+    const float d2 = d * d;
+    ssd = ssd + d2;
+  }
+  const float sd = sqrtf(ssd / cnt) + eps;
+  for (int64_t k = i; k < e; ++k) {
+    const float v = (r[k] - mean) / sd;
+    adv[k] = v;
+    if (adv2) adv2[k] = v;
+  }
+}
+
+// group_advantages with the group's rewards loaded by the 64 lanes of one wave at once
+// (chunks of 64), so the sequential sums run on registers instead of one dependent
+// load per reward: every lane forms the same sums from the same values in the same
+// order (readlane copies bits), hence the same bits as group_advantages. Called by all
+// 64 lanes of a wave.
+__device__ __forceinline__ void group_advantages_wave(const float* r, int64_t i, int64_t e, float eps, float* adv,
+                                                      float* adv2) {
+#pragma clang fp contract(off)
+  const int lane = threadIdx.x & 63;
+  const float cnt = static_cast<float>(e - i);
+  // Chunk c of 64 rewards: lane l holds r[i + 64 c + l]; the first chunk is kept.
+  const int n0 = static_cast<int>(min<int64_t>(64, e - i));
+  const float v0 = lane < n0 ? r[i + lane] : 0.f;
+  auto chunk = [&](int64_t c0) { return c0 == i ? v0 : (c0 + lane < e ? r[c0 + lane] : 0.f); };
+  float sum = 0.f;
+  for (int64_t c0 = i; c0 < e; c0 += 64) {
+    const int n = static_cast<int>(min<int64_t>(64, e - c0));
+    const float v = chunk(c0);
+    for (int k = 0; k < n; ++k) sum = sum + __shfl(v, k);
+  }
+  const float mean = sum / cnt;
+  float ssd = 0.f;
+  for (int64_t c0 = i; c0 < e; c0 += 64) {
+    const int n = static_cast<int>(min<int64_t>(64, e - c0));
+    const float v = chunk(c0);
+    for (int k = 0; k < n; ++k) {
+      const float d = __shfl(v, k) - mean;
+      const float d2 = d * d;
+      ssd = ssd + d2;
+    }
+  }
+  const float sd = sqrtf(ssd / cnt) + eps;
+  for (int64_t c0 = i; c0 < e; c0 += 64) {
+    if (c0 + lane >= e) break;
+    const float x = (chunk(c0) - mean) / sd;
+    adv[c0 + lane] = x;
+    if (adv2) adv2[c0 + lane] = x;
+  }
+}
+
+// The work before the row kernel in one launch, one workgroup per sequence s:
+//  * seq_len[s], seq_scale[s] as seq_prep_kernel (the same per-lane order and reduction);
+//  * with rewards: thread 0 of the first workgroup of each group computes the group's
+//    advantages as advantages_kernel (the same function, so the same bits), also into
+//    adv_out; without: adv_out[s] = adv_in[s] (when adv_out is set);
+//  * workgroup 0 zeroes the counters the row kernel and loss_reduce_kernel start from.
+__device__ __forceinline__ void step_prep(const StepPrepArgs& a, int64_t s, float* lds) {
+  // The mask terms first, in batches of four per lane with every load of a batch in
+  // flight before its additions (each lane still adds its terms in row order).
+  float acc = 0.f;
+  const int64_t base = s * a.tok_stride + a.tok_offset;
+  constexpr int kB = 4;
+  for (int64_t t0 = threadIdx.x; t0 < a.rows; t0 += kB * kSmallBlock) {
+    float m[kB];
+#pragma unroll
+    for (int q = 0; q < kB; ++q) {
+      const int64_t t = t0 + q * kSmallBlock;
+      m[q] = 1.f;
+      if (a.mask != nullptr && t < a.rows)
+        m[q] = a.mask_u8 ? (static_cast<const uint8_t*>(a.mask)[base + t] ? 1.f : 0.f)
+                         : static_cast<const float*>(a.mask)[base + t];
+    }
+#pragma unroll
+    for (int q = 0; q < kB; ++q)
+      if (t0 + q * kSmallBlock < a.rows) acc += m[q];
+  }
+  if (threadIdx.x == 0 && s == 0) {
+#pragma unroll
+    for (int k = 0; k < 3; ++k)
+      if (a.zero[k]) *a.zero[k] = 0;
+  }
+  if (a.rewards) {
+    if (s % a.group == 0 && threadIdx.x < 64)
+      group_advantages_wave(a.rewards, s, min(s + a.group, a.n_seq), a.std_eps, a.adv, a.adv_out);
+  } else if (a.adv_out && threadIdx.x == 0) {
+    a.adv_out[s] = a.adv_in[s];
+  }
+  const float tot = block_sum<kSmallBlock>(acc, lds);
+  if (threadIdx.x == 0) {
+    const float L = fmaxf(tot, 1.f);
+    a.seq_len[s] = L;
+    a.seq_scale[s] = 1.f / (a.loss_norm * L);
+  }
+}
+
+__global__ void __launch_bounds__(kSmallBlock) step_prep_kernel(StepPrepArgs a) {
+  __shared__ float lds[kSmallBlock / 64];
+  step_prep(a, blockIdx.x, lds);
+}
+
+// ---------------------------------------------------------------------------
+// Rows in parts (RowPlan::kParts), for launches with too few rows to fill the chip one
+// row to a workgroup: `parts` workgroups of 256 lanes take `per` <= 256 * kPartU 16-byte
+// vectors of a row each, one load per vector and all of them in flight at once. The first
+// kernel leaves each part's (max, sum) pairs; in the second every workgroup of a row
+// merges them for itself (the same values in the same order) and forms its part of
+// dlogits from a second read of the policy row, which a launch this small leaves in the
+// caches; forward-only calls have one wave per row merge instead. Rows off 16 bytes are
+// split as in grpo_fwd_kernel, part 0 taking the head and the tail. Every dlogit is the
+// f32 result rounded once. The first kernel, which needs neither lengths nor advantages,
+// also carries the loss's step_prep, so the loss takes no launch more than with a row to a
+// workgroup.
+// ---------------------------------------------------------------------------
+constexpr int kPartU = 8;
+constexpr int kPartBlock = 256;
+
+template <typename TI, bool REF>
+__global__ void __launch_bounds__(kPartBlock) grpo_part_kernel(RowArgs a, StepPrepArgs prep, int per) {
+  constexpr int EPV = 16 / TI::kBytes, U = kPartU, BLOCK = kPartBlock;
+  __shared__ __align__(16) float lds[4 * (BLOCK / 64)];
+  const int tid = threadIdx.x, part = blockIdx.x;
+  const int64_t row = blockIdx.y;
+  static_assert(kPartBlock == kSmallBlock, "step_prep's workgroup");
+  if (row >= a.nrows) {   // past the rows: one workgroup per sequence
+    if (part == 0) step_prep(prep, row - a.nrows, lds);
+    return;
+  }
+  const RowMeta r = row_meta(a, row);
+  if (!r.live) return;
+  const void* xrow = static_cast<const char*>(a.logits) + row * a.vocab * TI::kBytes;
+  const void* rrow = REF ? static_cast<const char*>(a.ref_logits) + row * a.vocab * TI::kBytes : nullptr;
+  const RowSpan xsp = row_span<TI>(xrow, a.vocab);
+  const RowSpan rsp = REF ? row_span<TI>(rrow, a.vocab) : xsp;
+  const int v0 = part * per, xend = min(v0 + per, xsp.nv), rend = min(v0 + per, rsp.nv);
+  const __amdgpu_buffer_rsrc_t xbuf = row_rsrc(xsp.vec, static_cast<uint32_t>(xend) * 16u);
+  const __amdgpu_buffer_rsrc_t rbuf = REF ? row_rsrc(rsp.vec, static_cast<uint32_t>(rend) * 16u) : xbuf;
+  const uint32_t off = static_cast<uint32_t>(v0 + tid) * 16u;
+  u32x4 xb[U], rb[U];
+#pragma unroll
+  for (int q = 0; q < U; ++q) xb[q] = buf_ld16<false>(xbuf, off + q * (BLOCK * 16u));   // read again for dlogits
+  if constexpr (REF) {
+#pragma unroll
+    for (int q = 0; q < U; ++q) rb[q] = buf_ld16<true>(rbuf, off + q * (BLOCK * 16u));
+  }
+  // One model's pair over this lane's vectors below lim, starting from its edge element.
+  auto pair = [&](const u32x4 (&b)[U], int lim, float& m, float& s) {
+    float bx = kNegInf;
+#pragma unroll
+    for (int q = 0; q < U; ++q)
+      if (v0 + q * BLOCK + tid < lim) bx = vec_max<TI>(bx, b[q]);
+    const float nm = fmaxf(m, bx * kLog2e), ref = ms_ref(nm);
+    float acc = ms_rescale(s, m, nm);
+#pragma unroll
+    for (int q = 0; q < U; ++q)
+      if (v0 + q * BLOCK + tid < lim) {
+        const uint32_t* w = reinterpret_cast<const uint32_t*>(&b[q]);
+#pragma unroll
+        for (int j = 0; j < EPV; ++j) acc += hw_exp2(fmaf(TI::unpack(w, j), kLog2e, -ref));
+      }
+    m = nm;
+    s = acc;
+  };
+  float pm = kNegInf, ps = 0.f, rm = kNegInf, rs = 0.f;
+  if (part == 0) {
+    edge_state<TI>(xrow, xsp, tid, pm, ps);
+    if constexpr (REF) edge_state<TI>(rrow, rsp, tid, rm, rs);
+  }
+  pair(xb, xend, pm, ps);
+  if constexpr (REF) pair(rb, rend, rm, rs);
+  block_merge2<BLOCK>(pm, ps, rm, rs, lds);
+  if (tid == 0) a.part[row * gridDim.x + part] = make_float4(pm, ps, rm, rs);
+}
+
+// The row's merged pairs (policy, reference) from its parts (at most 64), on every lane of
+// the wave.
+__device__ __forceinline__ float4 merge_parts(const RowArgs& a, int64_t row, int parts) {
+  const int lane = threadIdx.x & 63;
+  float4 w = make_float4(kNegInf, 0.f, kNegInf, 0.f);
+  if (lane < parts) w = a.part[row * parts + lane];
+  lanes_merge<64>(w.x, w.y);
+  lanes_merge<64>(w.z, w.w);
+  return w;
+}
+
+// Forward only: one wave per row.
+template <typename TI>
+__global__ void __launch_bounds__(64) grpo_part_merge_kernel(RowArgs a, int parts) {
+  const int64_t row = blockIdx.x;
+  const RowMeta r = row_meta(a, row);
+  if (!r.live) {
+    write_token_outputs(a, r, 0.f, 0.f, 0.f);
+    return;
+  }
+  const int64_t e = row * a.vocab + r.id;
+  const float xy = TI::load1(a.logits, e);
+  const float ry = a.ref_logits ? TI::load1(a.ref_logits, e) : 0.f;
+  const float4 w = merge_parts(a, row, parts);
+  const double lse = ms_lse(w.x, w.y), rlse = a.ref_logits ? ms_lse(w.z, w.w) : 0.;
+  flag_nonfinite(a, lse, rlse);
+  const double lp = xy - lse, lr = ry - rlse;
+  write_token_outputs(a, r, static_cast<float>(lp), static_cast<float>(lr), token_terms(a, r, lp, lr).loss);
+}
+
+template <typename TI, typename TO, int SP>
+__global__ void __launch_bounds__(kPartBlock) grpo_part_grad_kernel(RowArgs a, int per) {
+  constexpr int EPV = 16 / TI::kBytes, U = kPartU, BLOCK = kPartBlock;
+  constexpr uint32_t kOutVec = EPV * TO::kBytes;   // output bytes per input vector
+  const int tid = threadIdx.x, part = blockIdx.x;
+  const int64_t row = blockIdx.y, row_elem = row * a.vocab;
+  const RowMeta r = row_meta(a, row);
+  const void* xrow = static_cast<const char*>(a.logits) + row_elem * TI::kBytes;
+  const RowSpan xsp = row_span<TI>(xrow, a.vocab);   // the dlogits row splits alike
+  const int ek = part == 0 ? edge_index<TI>(xsp, tid) : -1;
+  const int v0 = part * per, end = min(v0 + per, xsp.nv);
+  // Loads and stores at or past this part's end fall outside the descriptors.
+  const uint32_t lim = static_cast<uint32_t>(end);
+  const __amdgpu_buffer_rsrc_t drow =
+      row_rsrc(static_cast<char*>(a.dlogits) + (row_elem + xsp.head) * TO::kBytes, lim * kOutVec);
+  if (!r.live) {
+    if (part == 0) write_token_outputs(a, r, 0.f, 0.f, 0.f);
+    if (a.zero_fill) {
+      const u32x4 z = {0u, 0u, 0u, 0u};
+#pragma unroll
+      for (int q = 0; q < U; ++q)
+#pragma unroll
+        for (uint32_t h = 0; h < kOutVec; h += 16)
+          buf_st16<true, SP>(drow, z, static_cast<uint32_t>(v0 + q * BLOCK + tid) * kOutVec + h);
+      if (ek >= 0) store1<TO>(a.dlogits, row_elem + ek, 0.f);
+    }
+    return;
+  }
+  const bool has_ref = a.ref_logits != nullptr;
+  const float xy = TI::load1(xrow, r.id);
+  const float ry = has_ref ? TI::load1(a.ref_logits, row_elem + r.id) : 0.f;
+  const float xe = ek >= 0 ? TI::load1(xrow, ek) : 0.f;
+  const __amdgpu_buffer_rsrc_t xbuf = row_rsrc(xsp.vec, lim * 16u);
+  u32x4 xb[U];
+#pragma unroll
+  for (int q = 0; q < U; ++q) xb[q] = buf_ld16<true>(xbuf, static_cast<uint32_t>(v0 + q * BLOCK + tid) * 16u);
+  const float4 mg = merge_parts(a, row, gridDim.x);
+  const float lse2 = mg.x + log2f(mg.y);
+  const double lse = ms_lse(mg.x, mg.y), rlse = has_ref ? ms_lse(mg.z, mg.w) : 0.;
+  const double lp = xy - lse, lr = ry - rlse;
+  const TokenTerms tt = token_terms(a, r, lp, lr);
+  if (part == 0) {
+    flag_nonfinite(a, lse, rlse);
+    write_token_outputs(a, r, static_cast<float>(lp), static_cast<float>(lr), tt.loss);
+  }
+  const float c = tt.coef, nc = -c;
+  const float dy = c - c * hw_exp2(fmaf(xy, kLog2e, -lse2));   // the target's own dlogit
+  const int64_t it = r.id - xsp.head;
+  const int tv = it >= 0 ? static_cast<int>(it / EPV) : -1, tj = static_cast<int>(it % EPV);
+#pragma unroll
+  for (int q = 0; q < U; ++q) {
+    const int vi = v0 + q * BLOCK + tid;
+    const uint32_t* w = reinterpret_cast<const uint32_t*>(&xb[q]);
+    float o[EPV];
+#pragma unroll
+    for (int j = 0; j < EPV; ++j) o[j] = nc * hw_exp2(fmaf(TI::unpack(w, j), kLog2e, -lse2));
+    if (vi == tv) {
+#pragma unroll
+      for (int j = 0; j < EPV; ++j)
+        if (j == tj) o[j] = dy;
+    }
+    buf_store_vals<TO, EPV, true, SP>(drow, static_cast<uint32_t>(vi) * kOutVec, o);
+  }
+  if (ek >= 0)
+    store1<TO>(a.dlogits, row_elem + ek, ek == r.id ? dy : nc * hw_exp2(fmaf(xe, kLog2e, -lse2)));
 }
 
 // ---------------------------------------------------------------------------
@@ -830,13 +1143,13 @@ __global__ void __launch_bounds__(BLOCK) grpo_stream_kernel(RowArgs a) {
 
   block_merge2<BLOCK>(pm, ps, rm, rs, lds);
   const float lse2 = pm + log2f(ps);
-  const float lse = lse2 * kLn2;
-  const float rlse = has_ref ? ms_lse(rm, rs) : 0.f;
+  const double lse = ms_lse(pm, ps);
+  const double rlse = has_ref ? ms_lse(rm, rs) : 0.;
   flag_nonfinite(a, lse, rlse);
-  const float lp = xy - lse;
-  const float lr = ry - rlse;
+  const double lp = xy - lse;
+  const double lr = ry - rlse;
   const TokenTerms tt = token_terms(a, r, lp, lr);
-  write_token_outputs(a, r, lp, lr, tt.loss);
+  write_token_outputs(a, r, static_cast<float>(lp), static_cast<float>(lr), tt.loss);
   if (a.dlogits == nullptr) return;
 
   const float c = tt.coef, nc = -tt.coef;
@@ -869,30 +1182,11 @@ __global__ void __launch_bounds__(BLOCK) grpo_stream_kernel(RowArgs a) {
 }
 
 // ---------------------------------------------------------------------------
-// Small kernels: sequence lengths, advantages, loss reduction.
+// Small kernels: the same as launches of their own, loss reduction.
 // ---------------------------------------------------------------------------
-
-// Deterministic workgroup sum: fixed per-lane order, xor butterfly (commutative,
-// so every lane agrees), fixed cross-wave order. Result on every thread.
-template <int BLOCK>
-__device__ __forceinline__ float block_sum(float v, float* lds) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off);
-  constexpr int NW = BLOCK / 64;
-  if constexpr (NW > 1) {
-    if ((threadIdx.x & 63) == 0) lds[threadIdx.x >> 6] = v;
-    __syncthreads();
-    v = lds[0];
-#pragma unroll
-    for (int w = 1; w < NW; ++w) v += lds[w];
-    __syncthreads();
-  }
-  return v;
-}
 
 // seq_len[s] = max(sum_t mask, 1)  (torch.clamp(shift_mask.sum(1), min=1.0),
 // export_qwen_forward.py:160); seq_scale[s] = 1 / (loss_norm * seq_len[s]).
-constexpr int kSmallBlock = 256;
 __global__ void __launch_bounds__(kSmallBlock)
 seq_prep_kernel(const void* mask, int32_t mask_u8, int64_t rows, int64_t tok_stride,
                 int64_t tok_offset, float loss_norm, float* seq_len, float* seq_scale) {
@@ -912,75 +1206,6 @@ seq_prep_kernel(const void* mask, int32_t mask_u8, int64_t rows, int64_t tok_str
     const float L = fmaxf(tot, 1.f);
     seq_len[s] = L;
     seq_scale[s] = 1.f / (loss_norm * L);
-  }
-}
-
-// Group-relative advantages, restating rl_shepherd.zig:466-478 operation by
-// operation in IEEE fp32: sequential sum, mean = sum / n, sequential sum of
-// (r-mean)*(r-mean), std = sqrt(ssd / n) + eps, (r-mean)/std. hipcc contracts
-// a*b+c into an FMA by default (also inside the __fmul_rn/__fadd_rn helpers,
-// which are compiled outside this scope), so the arithmetic is written with
-// plain operators under contract(off); fp32 '/' and sqrtf are correctly rounded
-// (hipcc's default -fhip-fp32-correctly-rounded-divide-sqrt).
-// The group of rewards [i, e): adv[k] (and adv2[k] when adv2 is not null).
-__device__ __forceinline__ void group_advantages(const float* r, int64_t i, int64_t e, float eps, float* adv,
-                                                 float* adv2) {
-#pragma clang fp contract(off)
-  const float cnt = static_cast<float>(e - i);
-  float sum = 0.f;
-  for (int64_t k = i; k < e; ++k) sum = sum + r[k];
-  const float mean = sum / cnt;
-  float ssd = 0.f;
-  for (int64_t k = i; k < e; ++k) {
-    const float d = r[k] - mean;
-    const float d2 = d * d;
-    ssd = ssd + d2;
-  }
-  const float sd = sqrtf(ssd / cnt) + eps;
-  for (int64_t k = i; k < e; ++k) {
-    const float v = (r[k] - mean) / sd;
-    adv[k] = v;
-    if (adv2) adv2[k] = v;
-  }
-}
-
-// group_advantages with the group's rewards loaded by the 64 lanes of one wave at once
-// (chunks of 64), so the sequential sums run on registers instead of one dependent
-// load per reward: every lane forms the same sums from the same values in the same
-// order (readlane copies bits), hence the same bits as group_advantages. Called by all
-// 64 lanes of a wave.
-__device__ __forceinline__ void group_advantages_wave(const float* r, int64_t i, int64_t e, float eps, float* adv,
-                                                      float* adv2) {
-#pragma clang fp contract(off)
-  const int lane = threadIdx.x & 63;
-  const float cnt = static_cast<float>(e - i);
-  // Chunk c of 64 rewards: lane l holds r[i + 64 c + l]; the first chunk is kept.
-  const int n0 = static_cast<int>(min<int64_t>(64, e - i));
-  const float v0 = lane < n0 ? r[i + lane] : 0.f;
-  auto chunk = [&](int64_t c0) { return c0 == i ? v0 : (c0 + lane < e ? r[c0 + lane] : 0.f); };
-  float sum = 0.f;
-  for (int64_t c0 = i; c0 < e; c0 += 64) {
-    const int n = static_cast<int>(min<int64_t>(64, e - c0));
-    const float v = chunk(c0);
-    for (int k = 0; k < n; ++k) sum = sum + __shfl(v, k);
-  }
-  const float mean = sum / cnt;
-  float ssd = 0.f;
-  for (int64_t c0 = i; c0 < e; c0 += 64) {
-    const int n = static_cast<int>(min<int64_t>(64, e - c0));
-    const float v = chunk(c0);
-    for (int k = 0; k < n; ++k) {
-      const float d = __shfl(v, k) - mean;
-      const float d2 = d * d;
-      ssd = ssd + d2;
-    }
-  }
-  const float sd = sqrtf(ssd / cnt) + eps;
-  for (int64_t c0 = i; c0 < e; c0 += 64) {
-    if (c0 + lane >= e) break;
-    const float x = (chunk(c0) - mean) / sd;
-    adv[c0 + lane] = x;
-    if (adv2) adv2[c0 + lane] = x;
   }
 }
 
@@ -1018,53 +1243,6 @@ loss_final_kernel(const float* seq_val, int64_t n_seq, float loss_norm, float* l
   for (int64_t s = threadIdx.x; s < n_seq; s += kFinalBlock) acc += seq_val[s];
   const float tot = block_sum<kFinalBlock>(acc, lds);
   if (threadIdx.x == 0) *loss = tot / loss_norm;
-}
-
-// The work before the row kernel in one launch, one workgroup per sequence s:
-//  * seq_len[s], seq_scale[s] as seq_prep_kernel (the same per-lane order and reduction);
-//  * with rewards: thread 0 of the first workgroup of each group computes the group's
-//    advantages as advantages_kernel (the same function, so the same bits), also into
-//    adv_out; without: adv_out[s] = adv_in[s] (when adv_out is set);
-//  * workgroup 0 zeroes the counters the row kernel and loss_reduce_kernel start from.
-__global__ void __launch_bounds__(kSmallBlock) step_prep_kernel(StepPrepArgs a) {
-  const int64_t s = blockIdx.x;
-  __shared__ float lds[kSmallBlock / 64];
-  // The mask terms first, in batches of four per lane with every load of a batch in
-  // flight before its additions (each lane still adds its terms in row order).
-  float acc = 0.f;
-  const int64_t base = s * a.tok_stride + a.tok_offset;
-  constexpr int kB = 4;
-  for (int64_t t0 = threadIdx.x; t0 < a.rows; t0 += kB * kSmallBlock) {
-    float m[kB];
-#pragma unroll
-    for (int q = 0; q < kB; ++q) {
-      const int64_t t = t0 + q * kSmallBlock;
-      m[q] = 1.f;
-      if (a.mask != nullptr && t < a.rows)
-        m[q] = a.mask_u8 ? (static_cast<const uint8_t*>(a.mask)[base + t] ? 1.f : 0.f)
-                         : static_cast<const float*>(a.mask)[base + t];
-    }
-#pragma unroll
-    for (int q = 0; q < kB; ++q)
-      if (t0 + q * kSmallBlock < a.rows) acc += m[q];
-  }
-  if (threadIdx.x == 0 && s == 0) {
-#pragma unroll
-    for (int k = 0; k < 3; ++k)
-      if (a.zero[k]) *a.zero[k] = 0;
-  }
-  if (a.rewards) {
-    if (s % a.group == 0 && threadIdx.x < 64)
-      group_advantages_wave(a.rewards, s, min(s + a.group, a.n_seq), a.std_eps, a.adv, a.adv_out);
-  } else if (a.adv_out && threadIdx.x == 0) {
-    a.adv_out[s] = a.adv_in[s];
-  }
-  const float tot = block_sum<kSmallBlock>(acc, lds);
-  if (threadIdx.x == 0) {
-    const float L = fmaxf(tot, 1.f);
-    a.seq_len[s] = L;
-    a.seq_scale[s] = 1.f / (a.loss_norm * L);
-  }
 }
 
 // The loss in one launch, one workgroup per sequence: seq_val[s] as seq_loss_kernel;
@@ -1197,6 +1375,27 @@ hipError_t launch_fwd(const RowArgs& a, int64_t nrows, hipStream_t st) {
   return hipGetLastError();
 }
 
+template <typename TI, typename TO>
+hipError_t launch_parts(const RowPlan& p, const RowArgs& a, const StepPrepArgs* prep, int64_t nrows, hipStream_t st) {
+  const int64_t nseq = prep ? prep->n_seq : 0;
+  if (nrows <= 0 || nrows != a.nrows || nrows + nseq > 65535 || a.part == nullptr || p.parts < 1 || p.parts > 64 || p.per > kPartBlock * kPartU)
+    return hipErrorInvalidValue;
+  const dim3 g(static_cast<unsigned>(p.parts), static_cast<unsigned>(nrows)), b(kPartBlock);
+  const dim3 g1(static_cast<unsigned>(p.parts), static_cast<unsigned>(nrows + nseq));
+  StepPrepArgs pa;
+  if (prep) pa = *prep;
+  else std::memset(&pa, 0, sizeof(pa));
+  if (a.ref_logits) grpo_part_kernel<TI, true><<<g1, b, 0, st>>>(a, pa, p.per);
+  else grpo_part_kernel<TI, false><<<g1, b, 0, st>>>(a, pa, p.per);
+  if (!a.dlogits)
+    grpo_part_merge_kernel<TI><<<dim3(static_cast<unsigned>(nrows)), dim3(64), 0, st>>>(a, p.parts);
+  else if (a.zero_fill)
+    grpo_part_grad_kernel<TI, TO, kBufNTSystem><<<g, b, 0, st>>>(a, p.per);
+  else
+    grpo_part_grad_kernel<TI, TO, kBufNT><<<g, b, 0, st>>>(a, p.per);
+  return hipGetLastError();
+}
+
 // Resident configurations: (BLOCK, NCH). A row of NV 16-byte vectors fits the
 // first configuration with BLOCK*NCH >= NV.
 struct ResCfg {
@@ -1248,16 +1447,35 @@ hipError_t dispatch_resident(int cfg, bool edge, bool exact, const RowArgs& a, i
 }
 
 template <typename TI, typename TO>
-hipError_t dispatch_rows(const RowPlan& p, const RowArgs& a, int64_t nrows, hipStream_t st) {
+hipError_t dispatch_rows(const RowPlan& p, const RowArgs& a, const StepPrepArgs* prep, int64_t nrows, hipStream_t st) {
   if (p.kind == RowPlan::kResident) return dispatch_resident<TI, TO>(p.cfg, p.edge != 0, p.exact != 0, a, nrows, st);
   if (p.kind == RowPlan::kForward) return launch_fwd<TI>(a, nrows, st);
+  if (p.kind == RowPlan::kParts) return launch_parts<TI, TO>(p, a, prep, nrows, st);
   if (p.kind == RowPlan::kStreamVec) return launch_stream<TI, TO, true>(a, nrows, st);
   return launch_stream<TI, TO, false>(a, nrows, st);
 }
 
 }  // namespace
 
-RowPlan plan_rows(int in_bytes, int64_t vocab, bool aligned16, bool edge_ok, bool forward_only, bool force_stream) {
+// Where few rows run in parts (kParts) and not one to a workgroup. Whole calls (clip-KL,
+// half of the rows live and the rest zero-filled unless said), us, a row to a workgroup |
+// in parts:
+//   bf16 151,936  16 rows  48 | 33   64  53 | 39   256  65 | 62   512 103 |  91   768 138 | 126   1024 163 | 161   1536 218 | 227
+//   bf16 100,000                     64  46 | 37   256  51 | 54   512  80 |  74   768 103 |  97   1024 120 | 120
+//   bf16  50,257                     64  38 | 34   256  43 | 44   512  60 |  56   768  74 |  68   1024  84 |  81
+//   bf16  32,768                     64  35 | 33   256  37 | 37   512  47 |  44                   1024  62 |  56
+//   bf16  16,384                     64 32.5 | 33.4 256 32.9 | 33.5                               1024  44 |  45
+//   f32  151,936 (streamed)          64  76 | 45   256  98 | 89   512 170 | 136   768 251 | 201   1024 323 | 269   1536 456 | 417
+//   bf16 151,936, no zero-fill, a fifth live       256  58 | 42   512  59 |  51   768  61 | 60
+// (f32 151,936, REINFORCE, 2048 rows: 414 | 435.) Log-probs of policy and reference, one
+// workgroup of 256 lanes per row | in parts:
+//   bf16 151,936  16 rows  55 | 35   64  55 | 39   256  57 | 48   512  68 |  57   1024 100 | 88   2048 132 | 125
+//   bf16  50,257 (policy)            64  30 | 29                  512  32 |  34   1024  38 | 38   2048  48 |  44
+constexpr int64_t kPartMinVecs = 4096, kPartMaxRows = 768, kPartMaxRowsStreamed = 1536;
+constexpr int64_t kPartMinVecsFwd = 12000, kPartMaxRowsFwd = 2048;
+
+RowPlan plan_rows(int in_bytes, int64_t vocab, bool aligned16, bool edge_ok, bool forward_only, bool force_stream,
+                  int64_t nrows) {
   RowPlan p;
   const int epv = 16 / in_bytes;
   const bool vec = aligned16 && (vocab % epv == 0);
@@ -1267,7 +1485,20 @@ RowPlan plan_rows(int in_bytes, int64_t vocab, bool aligned16, bool edge_ok, boo
   p.nch = 0;
   p.edge = 0;
   p.exact = 0;
+  p.parts = p.per = 0;
   if (force_stream) return p;
+  const int64_t nv = vocab / epv;   // the interior of a row off 16 bytes has at most as many
+  constexpr int64_t kVecs = kPartBlock * kPartU;
+  auto in_parts = [&](int64_t min_vecs, int64_t max_rows) {
+    const int64_t parts = (nv + kVecs - 1) / kVecs;
+    if (nv < min_vecs || parts > 64 || nrows > max_rows) return false;
+    p.kind = RowPlan::kParts;
+    p.block = kPartBlock;
+    p.parts = static_cast<int>(parts);
+    p.per = static_cast<int>((nv + parts - 1) / parts);
+    return true;
+  };
+  if (forward_only && in_parts(kPartMinVecsFwd, kPartMaxRowsFwd)) return p;
   // The forward kernel takes rows of any alignment. It addresses a row through a
   // 32-bit buffer offset that runs up to one batch past the row end: rows up to 2 GiB
   // take it, longer rows stream (64-bit addressing).
@@ -1280,7 +1511,7 @@ RowPlan plan_rows(int in_bytes, int64_t vocab, bool aligned16, bool edge_ok, boo
   // type and offset (the head and tail then line up); otherwise they stream.
   if (!vec && !edge_ok) return p;
 
-  const int64_t nv = vocab / epv;   // the interior of a row off 16 bytes has at most as many
+  if (!forward_only && in_parts(kPartMinVecs, kPartMaxRows)) return p;
   for (int i = 0; i < static_cast<int>(sizeof(kResCfgs) / sizeof(kResCfgs[0])); ++i) {
     if (static_cast<int64_t>(kResCfgs[i].block) * kResCfgs[i].nch >= nv) {
       p.kind = RowPlan::kResident;
@@ -1291,16 +1522,22 @@ RowPlan plan_rows(int in_bytes, int64_t vocab, bool aligned16, bool edge_ok, boo
       return p;
     }
   }
+  if (!forward_only) (void)in_parts(kPartMinVecs, kPartMaxRowsStreamed);
   return p;
 }
 
-hipError_t launch_rows(const RowPlan& p, int in_dtype, int out_dtype, const RowArgs& a,
+size_t plan_part_bytes(const RowPlan& p, int64_t nrows) {
+  return p.kind == RowPlan::kParts ? sizeof(float4) * static_cast<size_t>(nrows) * static_cast<size_t>(p.parts) : 0;
+}
+
+hipError_t launch_rows(const RowPlan& p, int in_dtype, int out_dtype, const RowArgs& a, const StepPrepArgs* prep,
                        int64_t nrows, hipStream_t st) {
-  if (in_dtype == PCP_BF16 && out_dtype == PCP_BF16) return dispatch_rows<BF16T, BF16T>(p, a, nrows, st);
-  if (in_dtype == PCP_BF16 && out_dtype == PCP_F32) return dispatch_rows<BF16T, F32T>(p, a, nrows, st);
-  if (in_dtype == PCP_F16 && out_dtype == PCP_F16) return dispatch_rows<F16T, F16T>(p, a, nrows, st);
-  if (in_dtype == PCP_F16 && out_dtype == PCP_F32) return dispatch_rows<F16T, F32T>(p, a, nrows, st);
-  if (in_dtype == PCP_F32 && out_dtype == PCP_F32) return dispatch_rows<F32T, F32T>(p, a, nrows, st);
+  if (prep && p.kind != RowPlan::kParts) return hipErrorInvalidValue;
+  if (in_dtype == PCP_BF16 && out_dtype == PCP_BF16) return dispatch_rows<BF16T, BF16T>(p, a, prep, nrows, st);
+  if (in_dtype == PCP_BF16 && out_dtype == PCP_F32) return dispatch_rows<BF16T, F32T>(p, a, prep, nrows, st);
+  if (in_dtype == PCP_F16 && out_dtype == PCP_F16) return dispatch_rows<F16T, F16T>(p, a, prep, nrows, st);
+  if (in_dtype == PCP_F16 && out_dtype == PCP_F32) return dispatch_rows<F16T, F32T>(p, a, prep, nrows, st);
+  if (in_dtype == PCP_F32 && out_dtype == PCP_F32) return dispatch_rows<F32T, F32T>(p, a, prep, nrows, st);
   return hipErrorInvalidValue;
 }
 

@@ -10,22 +10,26 @@ struct RowArgs;
 
 // Which row kernel serves a request.
 struct RowPlan {
-  enum Kind { kResident = 0, kStreamVec = 1, kStreamScalar = 2, kForward = 3 };
+  enum Kind { kResident = 0, kStreamVec = 1, kStreamScalar = 2, kForward = 3, kParts = 4 };
   int kind;
   int cfg;    // resident configuration index
   int block;  // lanes per workgroup
   int nch;    // resident 16-byte chunks per lane
   int edge;   // resident rows off 16 bytes (head / tail element-wise)
+  int parts;  // kParts: workgroups per row, and
+  int per;    //   16-byte vectors per workgroup
   int exact;  // bf16 -> bf16 resident rows without the f16 softmax cache (PCP_FLAG_EXACT_BF16)
 };
 
 // in_bytes: logits element size; aligned16: every row base is 16-byte aligned;
 // edge_ok: dlogits (if any) have the logits' element type and the same address mod 16,
-// so rows off 16 bytes split alike; forward_only: no dlogits are written.
-RowPlan plan_rows(int in_bytes, int64_t vocab, bool aligned16, bool edge_ok, bool forward_only, bool force_stream);
+// so rows off 16 bytes split alike; forward_only: no dlogits are written; nrows: rows of
+// the call (of the whole call where it runs in groups: a row's bits depend on the plan).
+RowPlan plan_rows(int in_bytes, int64_t vocab, bool aligned16, bool edge_ok, bool forward_only, bool force_stream,
+                  int64_t nrows);
+// Bytes of RowArgs::part that a plan needs for nrows rows (0 for every kind but kParts).
+size_t plan_part_bytes(const RowPlan& p, int64_t nrows);
 
-hipError_t launch_rows(const RowPlan& p, int in_dtype, int out_dtype, const RowArgs& a,
-                       int64_t nrows, hipStream_t st);
 hipError_t launch_seq_prep(const void* mask, int mask_u8, int64_t n_seq, int64_t rows,
                            int64_t tok_stride, int64_t tok_offset, float loss_norm,
                            float* seq_len, float* seq_scale, hipStream_t st);
@@ -55,6 +59,10 @@ struct StepPrepArgs {
   int* zero[3];           // optional counters set to 0
 };
 hipError_t launch_step_prep(const StepPrepArgs& a, hipStream_t st);
+
+// prep (kParts only, or nullptr): the loss's step prep, done by the same launches.
+hipError_t launch_rows(const RowPlan& p, int in_dtype, int out_dtype, const RowArgs& a, const StepPrepArgs* prep,
+                       int64_t nrows, hipStream_t st);
 
 // The loss in one launch (seq_loss_kernel + loss_final_kernel, the same summation
 // order): done must be 0 at the launch (step_prep_kernel zeroes it) and is left 0.

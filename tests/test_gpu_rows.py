@@ -284,3 +284,58 @@ def test_rows_past_the_first_grid(dtype, V, zero_fill, longest):
 
     for whole, own in zip(call(slice(0, S)), call(slice(S - 4, S))):
         assert torch.equal(whole[S - 4:], own)
+
+
+PARTS_CASES = [("bf16", 32768, "bf16"), ("bf16", 50257, "bf16"), ("bf16", 151936, "bf16"), ("bf16", 151937, "bf16"),
+               ("bf16", 65544, "f32"), ("bf16", 262152, "bf16"), ("f32", 16384, "f32"), ("f32", 50257, "f32"),
+               ("f32", 151936, "f32")]
+
+
+@pytest.mark.parametrize("zero_fill", [True, False])
+@pytest.mark.parametrize("dt,V,odt", PARTS_CASES, ids=[f"{c[0]}-{c[1]}-{c[2]}" for c in PARTS_CASES])
+def test_few_rows_in_parts_and_many_whole(dt, V, odt, zero_fill):
+    """Wide rows of a small call run in parts, each dlogit the f32 result rounded once; among more
+    rows (1,600 here) the same rows run one to a workgroup (or stream). Both against the oracle:
+    the narrowest vocabularies in parts, ragged last parts, rows off 16 bytes, a shifted layout,
+    targets in the first and the last vector and in the head and tail, dead and ignored rows."""
+    rng = np.random.default_rng(V + len(odt))
+    S, T = 3, 5
+    rows, off = T - 1, 1
+    x32 = rng.standard_normal((S, T, V)).astype(np.float32) * 3
+    r32 = x32 + rng.standard_normal((S, T, V)).astype(np.float32) * 0.1
+    x, ref, code = (x32, r32, orc.F32) if dt == "f32" else (orc.bf16_from_f32(x32), orc.bf16_from_f32(r32), orc.BF16)
+    ids = rng.integers(0, V, size=(S, T)).astype(np.int64)
+    ids[0, 1:] = [0, V - 1, V // 2, 7]
+    ids[1, 2] = -100
+    mask = (np.arange(T)[None] < np.array([5, 5, 3])[:, None]).astype(np.float32)
+    adv = np.array([0.75, -1.25, 0.5], np.float32)
+    old = np.zeros((S, T), np.float32)
+    lp, _ = orc.logprob(np.ascontiguousarray(x[:, :rows]).reshape(S * rows, V), np.clip(ids[:, 1:].reshape(-1), 0, None),
+                        dtype=code)
+    old[:, 1:] = lp.reshape(S, rows) + rng.standard_normal((S, rows)) * 0.05
+    want = orc.grpo_full(x, ids, mask, rows=rows, tok_offset=off, advantages_in=adv, ref_logits=ref, old_logp=old,
+                         loss_mode=orc.CLIP_KL, loss_norm=3.0, dtype=code)
+    ts = token_scale(x, ids, rows, off, code)
+    fl = tok_to_rows(full_floor(want, mask, old, S, False, 0.04, 0.2, ts), rows, off, T)
+    dead = np.ones((S, T), bool)
+    dead[:, :rows] = (mask[:, 1:] == 0) | (ids[:, 1:] == -100)
+    tdt = {"bf16": torch.bfloat16, "f32": torch.float32}[odt]
+
+    def padded(a, n):   # n - S sequences of masked tokens after the case's own
+        a = dev(a)
+        return torch.cat([a, torch.zeros((n - S, *a.shape[1:]), dtype=a.dtype, device=DEV)])
+
+    for n in (S, 320):
+        print(f"rows in parts / whole: {dt}->{odt} V={V} sequences={n} zero_fill={zero_fill}", flush=True)
+        dl = torch.full((n, T, V), -3.5, dtype=tdt, device=DEV)
+        out = grpo.grpo_loss_fwd_bwd(padded(x, n), padded(ids, n), padded(mask, n), advantages=padded(adv, n),
+                                     ref_logits=padded(ref, n), old_logp=padded(old, n), rows=rows, tok_offset=off,
+                                     loss_mode=LossMode.GRPO_CLIP_KL, loss_norm=3.0, dlogits=dl, zero_fill=zero_fill)
+        assert np.all(np.abs(out.logp[:S].cpu().numpy()[:, 1:] - want.lp[:, 1:]) <= 1e-5 * ts[:, 1:])
+        assert abs(float(out.loss.cpu()) - want.loss) <= full_loss_tol(want, x, ids, mask, rows, off, code, False,
+                                                                       0.04, S)
+        bits = host_bits(out.dlogits[:S])
+        got = orc.bf16_to_f32(bits) if odt == "bf16" else bits
+        assert_dlogits(got[~dead], want.dlogits[~dead], fl[~dead], odt == "bf16", exact=n == S)
+        fill = 0.0 if zero_fill else -3.5
+        assert np.all(got[dead] == fill) and bool((dl[S:] == fill).all())
