@@ -118,11 +118,11 @@ struct LmDcacheArgs {
 };
 
 struct LmReduceArgs {
-  const float2* part;
+  const float2* part[2];  // per model; part[1] nullptr: one model
   int64_t N;              // bounds *count (the grid)
   const int* count;       // [1] live tokens (device)
   int ldp, nvt;
-  float* lse2;          // out
+  float* lse2[2];         // out
 };
 
 struct LmTermsArgs {

@@ -331,9 +331,9 @@ int run_lm(pcp_ctx* ctx, const pcp_lmhead_args* a) {
     if (timed && (e = hipEventRecord(ctx->prof_stop[ctx->prof_used++], st)) != hipSuccess)
       return hip_fail(ctx, e, "hipEventRecord");
   }
-  for (int m = 0; m < (ref ? 2 : 1); ++m) {
-    const LmReduceArgs rd{m == 0 ? part : reinterpret_cast<float2*>(sp + o_part2), N, cnt, npart, npart,
-                          F(m == 0 ? o_l2 : o_rl2)};
+  {
+    const LmReduceArgs rd{{part, ref ? reinterpret_cast<float2*>(sp + o_part2) : nullptr}, N, cnt, npart, npart,
+                          {F(o_l2), F(o_rl2)}};
     if ((e = launch_lm_reduce(rd, st)) != hipSuccess) return hip_fail(ctx, e, "LM-head reduce");
   }
 
