@@ -88,6 +88,30 @@ def test_base64_rejects_what_std_base64_rejects(bad):
     assert e.value.code == -1
 
 
+def test_base64_every_byte_value():
+    """Every byte value as a character at every place of the fast kernel's 16-character unit:
+    accepted exactly if it is in the alphabet, and then decoded as Python does; and every 6-bit
+    value encoded at every place."""
+    alphabet = b"ABCDEFGHIJKLMNOPQRSTUVWXYZabcdefghijklmnopqrstuvwxyz0123456789+/"
+    rng = np.random.default_rng(5)
+    for c in range(256):
+        ok = c in alphabet
+        for place in range(16):
+            text = bytearray(rng.choice(list(alphabet), 64).astype(np.uint8).tobytes())
+            text[16 + place] = c
+            if not ok and place % 5 != c % 5:
+                continue
+            dev_text = torch.from_numpy(np.frombuffer(bytes(text), np.uint8).copy()).to(DEV)
+            if ok:
+                assert formats.b64decode(dev_text).cpu().numpy().tobytes() == base64.b64decode(bytes(text))
+            else:
+                with pytest.raises(PcpError) as e:
+                    formats.b64decode(dev_text)
+                assert e.value.code == -1
+    words = base64.b64decode(bytes(alphabet[(i + k) % 64] for k in range(16) for i in range(64)))
+    assert formats.b64encode(torch.from_numpy(np.frombuffer(words, np.uint8).copy()).to(DEV)).cpu().numpy().tobytes() == base64.b64encode(words)
+
+
 def test_update_weights_payload_full_size():
     """The UPDATE_WEIGHTS payload of Qwen2.5-0.5B's 494,032,768 f32 weights (1.98 GB):
     encoded on the device and decoded back bit for bit; a sample checked against Python."""
