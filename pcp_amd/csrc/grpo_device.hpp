@@ -388,7 +388,8 @@ struct RowArgs {
   // rows. nullptr: every row in order.
   int* row_list;
   int* row_count;
-  float4* part;            // RowPlan::kParts: [nrows, parts] (policy m, s, reference m, s)
+  float4* part;            // RowPlan::kParts: [nrows, parts] (policy m, s, reference m, s), then
+                           // [nrows] (the target's policy and reference logits)
   int64_t nrows;           // logits rows of the launch
   int64_t vocab;
   int64_t rows;

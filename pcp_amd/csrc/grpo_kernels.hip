@@ -876,7 +876,9 @@ __global__ void __launch_bounds__(kSmallBlock) step_prep_kernel(StepPrepArgs a) 
 // dlogits from a second read of the policy row, which a launch this small leaves in the
 // caches; forward-only calls have one wave per row merge instead. Rows off 16 bytes are
 // split as in grpo_fwd_kernel, part 0 taking the head and the tail. Every dlogit is the
-// f32 result rounded once. The first kernel, which needs neither lengths nor advantages,
+// f32 result rounded once. dlogits may be the logits themselves, as with a row to a
+// workgroup: a part reads its own vectors before it writes them, and the target's logit,
+// which may lie in another part, comes from the first kernel. The first kernel, which needs neither lengths nor advantages,
 // also carries the loss's step_prep, so the loss takes no launch more than with a row to a
 // workgroup.
 // ---------------------------------------------------------------------------
@@ -937,7 +939,12 @@ __global__ void __launch_bounds__(kPartBlock) grpo_part_kernel(RowArgs a, StepPr
   pair(xb, xend, pm, ps);
   if constexpr (REF) pair(rb, rend, rm, rs);
   block_merge2<BLOCK>(pm, ps, rm, rs, lds);
-  if (tid == 0) a.part[row * gridDim.x + part] = make_float4(pm, ps, rm, rs);
+  if (tid == 0) {
+    a.part[row * gridDim.x + part] = make_float4(pm, ps, rm, rs);
+    if (part == 0)   // the target's logits, which dlogits written in place may replace
+      a.part[a.nrows * gridDim.x + row] =
+          make_float4(TI::load1(xrow, r.id), REF ? TI::load1(rrow, r.id) : 0.f, 0.f, 0.f);
+  }
 }
 
 // The row's merged pairs (policy, reference) from its parts (at most 64), on every lane of
@@ -999,8 +1006,8 @@ __global__ void __launch_bounds__(kPartBlock) grpo_part_grad_kernel(RowArgs a, i
     return;
   }
   const bool has_ref = a.ref_logits != nullptr;
-  const float xy = TI::load1(xrow, r.id);
-  const float ry = has_ref ? TI::load1(a.ref_logits, row_elem + r.id) : 0.f;
+  const float4 target = a.part[a.nrows * gridDim.x + row];
+  const float xy = target.x, ry = target.y;
   const float xe = ek >= 0 ? TI::load1(xrow, ek) : 0.f;
   const __amdgpu_buffer_rsrc_t xbuf = row_rsrc(xsp.vec, lim * 16u);
   u32x4 xb[U];
@@ -1527,7 +1534,7 @@ RowPlan plan_rows(int in_bytes, int64_t vocab, bool aligned16, bool edge_ok, boo
 }
 
 size_t plan_part_bytes(const RowPlan& p, int64_t nrows) {
-  return p.kind == RowPlan::kParts ? sizeof(float4) * static_cast<size_t>(nrows) * static_cast<size_t>(p.parts) : 0;
+  return p.kind == RowPlan::kParts ? sizeof(float4) * static_cast<size_t>(nrows) * static_cast<size_t>(p.parts + 1) : 0;
 }
 
 hipError_t launch_rows(const RowPlan& p, int in_dtype, int out_dtype, const RowArgs& a, const StepPrepArgs* prep,

@@ -339,3 +339,21 @@ def test_few_rows_in_parts_and_many_whole(dt, V, odt, zero_fill):
         assert_dlogits(got[~dead], want.dlogits[~dead], fl[~dead], odt == "bf16", exact=n == S)
         fill = 0.0 if zero_fill else -3.5
         assert np.all(got[dead] == fill) and bool((dl[S:] == fill).all())
+
+
+@pytest.mark.parametrize("dt,V", [("bf16", 50257), ("bf16", 151936), ("f32", 50257)])
+def test_rows_in_parts_in_place(dt, V):
+    """dlogits written over the logits: the same bits as into a buffer of their own, with targets
+    in every part of the row and in its head and tail."""
+    gen = torch.Generator(device=DEV).manual_seed(V)
+    S, T = 4, 48
+    x = (torch.randn((S, T, V), generator=gen, device=DEV) * 3).to({"bf16": torch.bfloat16, "f32": torch.float32}[dt])
+    ref = (x.float() + 0.1 * torch.randn((S, T, V), generator=gen, device=DEV)).to(x.dtype)
+    ids = torch.linspace(0, V - 1, S * T, device=DEV).long().view(S, T)
+    mask = (torch.arange(T, device=DEV)[None] < torch.tensor([[48], [31], [48], [9]], device=DEV)).float()
+    kw = dict(advantages=torch.tensor([0.75, -1.25, 0.5, 1.0], device=DEV), ref_logits=ref,
+              old_logp=-torch.rand((S, T), generator=gen, device=DEV) * 9, loss_mode=LossMode.GRPO_CLIP_KL)
+    want = grpo.grpo_loss_fwd_bwd(x, ids, mask, dlogits=torch.empty_like(x), **kw)
+    got = grpo.grpo_loss_fwd_bwd(x, ids, mask, dlogits=x, **kw)
+    for f in ("loss", "dlogits", "logp", "ref_logp", "token_loss"):
+        assert torch.equal(getattr(got, f), getattr(want, f)), f
