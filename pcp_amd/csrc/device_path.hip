@@ -230,7 +230,9 @@ int run(pcp_ctx* ctx, const pcp_grpo_args* a, Op op, bool noalloc = false, int64
     plan = plan_for(INT64_MAX);   // no room for the parts' results: a row per workgroup
     part_bytes = 0;
   }
-  const size_t need = 4 * sv + 512 + tl_bytes + list_bytes + part_bytes;
+  // The context's buffer always has room for any call's parts, so that a call of fewer rows
+  // than the one before it, which may run in parts where that did not, needs no more of it.
+  const size_t need = 4 * sv + 512 + tl_bytes + list_bytes + (noalloc ? part_bytes : kPartScratchBytes);
   if (noalloc && need > PCP_NOALLOC_SCRATCH_BYTES)
     return fail(ctx, PCP_ERR_OVERFLOW,
                 "the allocation-free call needs %zu bytes of work space, more than its %u-byte array: pass "

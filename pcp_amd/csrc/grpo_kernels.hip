@@ -1480,6 +1480,7 @@ hipError_t dispatch_rows(const RowPlan& p, const RowArgs& a, const StepPrepArgs*
 //   bf16  50,257 (policy)            64  30 | 29                  512  32 |  34   1024  38 | 38   2048  48 |  44
 constexpr int64_t kPartMinVecs = 4096, kPartMaxRows = 768, kPartMaxRowsStreamed = 1536;
 constexpr int64_t kPartMinVecsFwd = 12000, kPartMaxRowsFwd = 2048;
+static_assert(kPartScratchBytes == sizeof(float4) * kPartMaxRowsFwd * (64 + 1), "the largest launch in parts");
 
 RowPlan plan_rows(int in_bytes, int64_t vocab, bool aligned16, bool edge_ok, bool forward_only, bool force_stream,
                   int64_t nrows) {

@@ -27,7 +27,9 @@ struct RowPlan {
 // the call (of the whole call where it runs in groups: a row's bits depend on the plan).
 RowPlan plan_rows(int in_bytes, int64_t vocab, bool aligned16, bool edge_ok, bool forward_only, bool force_stream,
                   int64_t nrows);
-// Bytes of RowArgs::part that a plan needs for nrows rows (0 for every kind but kParts).
+// Bytes of RowArgs::part that a plan needs for nrows rows (0 for every kind but kParts), and
+// their upper bound: 2,048 rows of 64 parts.
+constexpr size_t kPartScratchBytes = 2048 * (64 + 1) * 16;
 size_t plan_part_bytes(const RowPlan& p, int64_t nrows);
 
 hipError_t launch_seq_prep(const void* mask, int mask_u8, int64_t n_seq, int64_t rows,

@@ -26,6 +26,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdint>
 #include <cstring>
 
@@ -171,19 +172,33 @@ int run_lm(pcp_ctx* ctx, const pcp_lmhead_args* a) {
   const int64_t ldt_max = (N + 63) / 64 * 64 + ((N + 63) / 64 * 64 % 256 == 0 ? 64 : 0);
   const size_t o_ht = a->dweight ? take(2 * static_cast<size_t>(H) * ldt_max) : 0;
   // The cached backward's products in K pieces (lm_ksplit): dhidden's pieces are compact
-  // [N, H] buffers one after the other, dW's [V, H] ones (at most 2 x 256 CUs' worth of
-  // 256 x 256 f32 tiles in all, 134 MB). A tile's prologue and epilogue count as four stages.
-  const int64_t nht = (H + kLmTileT - 1) / kLmTileT, ntk = (N + kLmTileV - 1) / kLmTileV;
-  const int64_t sd = (V + 63) / 64 + 4, sw = (N + 63) / 64 + 4;
-  const bool may_split = bwd && a->vocab_chunk == 0;
-  const int split_d = may_split && want_dy ? lm_ksplit(ntk * nht, sd, a->dweight ? nvt * nht * sw : 0) : 1;
-  const int split_w = may_split && a->dweight ? lm_ksplit(nvt * nht, sw, want_dy ? ntk * nht * sd : 0) : 1;
-  const size_t o_dhc = want_dy ? take(4 * static_cast<size_t>(N) * H * split_d) : 0;
-  const size_t o_dwp = split_w > 1 ? take(4 * static_cast<size_t>(V) * H * split_w) : 0;
+  // [N, H] buffers one after the other, dW's [V, H] ones. A tile's prologue and epilogue
+  // count as four stages. The pieces have room at the end for every call of up to N tokens
+  // (their number falls as N grows), so that a call of fewer tokens than the one before it
+  // needs no larger buffer; without memory for them the tiles stay whole.
+  const int64_t nht = (H + kLmTileT - 1) / kLmTileT, sd = (V + 63) / 64 + 4;
+  int split_d = 1, split_w = 1;
+  size_t d_bytes = 0, piece_bytes = 0;   // dhidden's pieces of this call; all of the largest call's
+  if (bwd && a->vocab_chunk == 0) {
+    for (int64_t s = 1; s <= (N + 63) / 64; ++s) {
+      const int64_t n = s * 64 < N ? s * 64 : N, ntk = (n + kLmTileV - 1) / kLmTileV, sw = s + 4;
+      split_d = want_dy ? lm_ksplit(ntk * nht, sd, a->dweight ? nvt * nht * sw : 0) : 1;
+      split_w = a->dweight ? lm_ksplit(nvt * nht, sw, want_dy ? ntk * nht * sd : 0) : 1;
+      d_bytes = split_d > 1 ? r256(4 * static_cast<size_t>(n) * H * split_d) : 0;
+      piece_bytes = std::max(piece_bytes, d_bytes + (split_w > 1 ? 4 * static_cast<size_t>(V) * H * split_w : 0));
+    }
+  }
+  const size_t o_dhc_whole = want_dy ? take(4 * static_cast<size_t>(N) * H) : 0;
   const size_t o_rstd = norm ? take(4 * N) : 0;
   const size_t o_gpart = a->dnorm_weight ? take(4 * static_cast<size_t>(kLmNormSlices) * H) : 0;
+  const size_t whole = off, o_pieces = take(piece_bytes);
   rc = ensure_scratch(ctx, off);
+  if (rc == PCP_ERR_OOM && piece_bytes) {
+    split_d = split_w = 1;
+    rc = ensure_scratch(ctx, whole);
+  }
   if (rc != PCP_OK) return rc;
+  const size_t o_dhc = split_d > 1 ? o_pieces : o_dhc_whole, o_dwp = o_pieces + d_bytes;
   char* sp = static_cast<char*>(ctx->scratch);
   auto F = [&](size_t o) { return reinterpret_cast<float*>(sp + o); };
   auto I = [&](size_t o) { return reinterpret_cast<int*>(sp + o); };

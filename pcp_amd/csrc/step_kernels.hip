@@ -420,9 +420,13 @@ int pcp_grad_stats_compute_many(pcp_ctx* ctx, int n_tensors, const float* const*
   hipStream_t st = static_cast<hipStream_t>(stream);
   StatsPart h{0.0, 0.f, 0, 0, 0};
   if (elements > 0) {
-    // A launch takes up to kStatsTensors tensors and writes at most kStatsBlocks partials.
+    // A launch takes up to kStatsTensors tensors and writes at most kStatsBlocks partials,
+    // fewer with more than 16 launches: the context's buffer, which a captured graph may
+    // hold, is never below 1 MB and then does not grow for them.
     const int64_t launches = (n_tensors + kStatsTensors - 1) / kStatsTensors;
-    const int64_t cap = chunks < launches * kStatsBlocks ? chunks : launches * kStatsBlocks;
+    const int64_t room = (1 << 20) / sizeof(StatsPart) / launches;
+    const int blocks = room > kStatsBlocks ? kStatsBlocks : room > 1 ? static_cast<int>(room) : 1;
+    const int64_t cap = chunks < launches * blocks ? chunks : launches * blocks;
     int rc = ensure_scratch(ctx, sizeof(StatsPart) * static_cast<size_t>(cap));
     if (rc != PCP_OK) return rc;
     StatsPart* parts = static_cast<StatsPart*>(ctx->scratch);
@@ -439,7 +443,7 @@ int pcp_grad_stats_compute_many(pcp_ctx* ctx, int n_tensors, const float* const*
         ++b.tensors;
       }
       if (b.tensors == 0) break;
-      const int n = b.first[b.tensors], grid = n < kStatsBlocks ? n : kStatsBlocks;
+      const int n = b.first[b.tensors], grid = n < blocks ? n : blocks;
       stats_kernel<<<grid, 256, 0, st>>>(b, parts + nparts);
       nparts += grid;
     }

@@ -1069,3 +1069,39 @@ def test_lmhead_large_batch_cached_matches_chunked():
         worst = float((a - b).abs().max() / b.abs().max())
         print(f"  low-memory {name}: relative Frobenius difference {rel:.2e}, largest {worst:.2e}", flush=True)
         assert bool(torch.isfinite(a).all()) and rel < 2 ** -16 and worst < 2 ** -12, (name, rel, worst)
+
+
+def test_captured_after_a_call_of_more_tokens():
+    """Fewer tokens can be cut into more K pieces (4,353 tokens into 15, 4,352 into 16 here); the
+    buffers that a larger call left still hold them, so the smaller call can be captured."""
+    H, V = 256, 20000
+    gen = torch.Generator(device="cuda:0").manual_seed(3)
+
+    def call(n, ctx, **kw):
+        return grpo.lmhead_fwd_bwd(hidden[:n], weight, ids[:, :n].contiguous(), mask[:, :n].contiguous(),
+                                   advantages=adv, loss_mode=LossMode.REINFORCE, ctx=ctx, **kw)
+
+    hidden = torch.randn((4353, H), generator=gen, device="cuda:0").to(torch.bfloat16)
+    weight = (torch.randn((V, H), generator=gen, device="cuda:0") * 0.1).to(torch.bfloat16)
+    ids = torch.randint(0, V, (1, 4353), generator=gen, device="cuda:0")
+    mask, adv = torch.ones((1, 4353), device="cuda:0"), torch.ones(1, device="cuda:0")
+    ctx = grpo.Context(0)
+    call(4353, ctx)
+    held = ctx.workspace_bytes()
+    want = call(4352, ctx)
+    assert ctx.workspace_bytes() == held
+    out = call(4352, ctx)
+    args = (hidden[:4352], weight, ids[:, :4352].contiguous(), mask[:, :4352].contiguous())
+    g = torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(g):
+        grpo.lmhead_fwd_bwd(*args, advantages=adv, loss_mode=LossMode.REINFORCE, outputs=out, sync=False, ctx=ctx)
+    for rep in range(3):
+        for f in ("loss", "logp", "dhidden", "dweight"):
+            getattr(out, f).fill_(float("nan"))
+        print(f"graph replay {rep}", flush=True)
+        g.replay()
+        torch.cuda.synchronize()
+        for f in ("loss", "logp", "dhidden", "dweight"):
+            assert torch.equal(getattr(out, f), getattr(want, f)), (rep, f)
+    ctx.sync()
