@@ -193,10 +193,10 @@ const char* pcp_last_error(const pcp_ctx* ctx);
 int pcp_sync(pcp_ctx* ctx);
 /* Free the context's grow-only device work buffers: the per-call scratch and the
  * LM-head backward workspace (the softmax cache: 11.3 GB at 16,384 tokens, V =
- * 151,936, H = 4,096; 21.4 GB with PCP_FLAG_EXACT_BF16), which otherwise stay held
- * until pcp_destroy. Synchronises the device first (every stream: calls enqueued with
- * PCP_FLAG_ASYNC may still use the buffers). The next call allocates again. No
- * counterpart in the reference (IREE holds its own device pools). */
+ * 151,936, H = 4,096; 21.4 GB with PCP_FLAG_EXACT_BF16; partial products of short calls),
+ * which otherwise stay held until pcp_destroy. Synchronises the device first (every
+ * stream: calls enqueued with PCP_FLAG_ASYNC may still use the buffers). The next call
+ * allocates again. No counterpart in the reference (IREE holds its own device pools). */
 int pcp_release_workspace(pcp_ctx* ctx);
 /* Bytes of device work buffers the context holds now (0 for NULL). */
 size_t pcp_workspace_bytes(const pcp_ctx* ctx);
@@ -310,7 +310,11 @@ int pcp_grpo_loss_fwd_bwd_noalloc(pcp_ctx* ctx, const pcp_grpo_args* a);
  * logit tiles per vocab chunk instead (dlogits = the f32 value rounded once): with a
  * transposed copy of the chunk and of the weight (2 * (2 * tokens * chunk + hidden *
  * vocab) bytes, within the same budget), or, when that does not fit, in memory
- * bounded by the chunk alone (2 * tokens * chunk bytes).
+ * bounded by the chunk alone (2 * tokens * chunk bytes). On the cached path products with
+ * few tiles are summed from partial products (under 300 MB, by the same rule of half the
+ * free memory); a call that was refused them, and those of its size after it until
+ * pcp_release_workspace, form the products in one piece, several times slower with few
+ * tokens, in another order of summation.
  * The live-token count never leaves the device: with PCP_FLAG_ASYNC the call only
  * enqueues work, and it can be captured in a HIP graph. A captured graph uses the
  * context's work buffers as they were at capture: make one uncaptured call of the same

@@ -478,6 +478,7 @@ void pcp_destroy(pcp_ctx* ctx) {
     release_profile_events(ctx);
     if (ctx->scratch) (void)hipFree(ctx->scratch);
     if (ctx->lm_dbuf) (void)hipFree(ctx->lm_dbuf);
+    if (ctx->lm_pieces.buf) (void)hipFree(ctx->lm_pieces.buf);
     if (ctx->sample_ticket) (void)hipFree(ctx->sample_ticket);
     destroy_stager(ctx);
     for (hipStream_t x : ctx->xs)
@@ -492,17 +493,22 @@ int pcp_release_workspace(pcp_ctx* ctx) {
   if (!ctx) return fail(nullptr, PCP_ERR_INVALID_ARG, "context is NULL");
   hipError_t e = hipSetDevice(ctx->device);
   if (e != hipSuccess) return hip_fail(ctx, e, "hipSetDevice");
-  if (!ctx->scratch && !ctx->lm_dbuf) return PCP_OK;
+  if (!ctx->scratch && !ctx->lm_dbuf && !ctx->lm_pieces.buf) {
+    ctx->lm_pieces.reset();
+    return PCP_OK;
+  }
   // Earlier calls (PCP_FLAG_ASYNC ones included) may still use the buffers.
   if ((e = hipDeviceSynchronize()) != hipSuccess) return hip_fail(ctx, e, "hipDeviceSynchronize");
   if (ctx->scratch) (void)hipFree(ctx->scratch);
   if (ctx->lm_dbuf) (void)hipFree(ctx->lm_dbuf);
+  if (ctx->lm_pieces.buf) (void)hipFree(ctx->lm_pieces.buf);
+  ctx->lm_pieces.reset();
   ctx->scratch = ctx->lm_dbuf = nullptr;
   ctx->scratch_bytes = ctx->lm_dbuf_bytes = 0;
   return PCP_OK;
 }
 
-size_t pcp_workspace_bytes(const pcp_ctx* ctx) { return ctx ? ctx->scratch_bytes + ctx->lm_dbuf_bytes : 0; }
+size_t pcp_workspace_bytes(const pcp_ctx* ctx) { return ctx ? ctx->scratch_bytes + ctx->lm_dbuf_bytes + ctx->lm_pieces.bytes : 0; }
 
 int pcp_get_backend_type(const pcp_ctx* ctx) { return ctx ? ctx->backend : PCP_ERR_INVALID_ARG; }
 

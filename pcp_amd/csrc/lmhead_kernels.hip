@@ -1503,31 +1503,6 @@ hipError_t launch_lm_sum_parts(const float* src, int nsplit, int64_t stride, flo
   return hipGetLastError();
 }
 
-// The cached backward's dhidden has few, long tiles (one per 256 tokens x 256 hidden
-// columns, K = the vocabulary: 2374 stages at V = 151,936), dW many short ones, so with
-// few tokens a handful of CUs ran dhidden for milliseconds after dW was done: 288 live
-// tokens at H = 896 took 2.89 ms for the launch, 8 CUs busy. A product whose tile is longer
-// than half of a CU's even share of the launch is therefore cut along K into pieces of
-// half that share (the share counts every token, and about half of them are live, so a
-// piece is then a CU's live share), at least 16 stages (below that a piece's f32 tile
-// costs more than its products). Each piece stores its own f32 partial tile, and the pieces
-// are added in order, so results stay deterministic. Whole calls, ms, before and with
-// pieces of 1/2, 1/4, 1/8 and 1/16 of the share (tokens x H x V):
-//    64 x  256 x 151936  3.70 |  .254  .253  .254  .251
-//   512 x  896 x 151936  3.39 |  .740  .745  .785  .800
-//  1024 x 4096 x 151936  5.30 |  3.12  3.09  3.12  3.17
-//  2048 x 2048 x  50257  1.70 |  1.02  1.03  1.07  1.14
-//  4096 x  896 x 151936  4.60 |  2.60  2.63  2.65  2.70
-// 16384 x  256 x   1000  .319 |  .165  .166  .165  .165   (here dW is the long one)
-// Configuration 5 (its dhidden tiles are an eighth of the share) stays whole.
-int lm_ksplit(int64_t tiles, int64_t stages, int64_t other) {
-  constexpr int64_t kCus = 256, kMin = 16;
-  const int64_t share = (tiles * stages + other) / kCus;   // stages per CU, evenly dealt
-  if (tiles <= 0 || 2 * stages <= share) return 1;
-  const int64_t piece = share / 2 > kMin ? share / 2 : kMin;
-  return static_cast<int>((stages + piece - 1) / piece);
-}
-
 hipError_t launch_lm_zero(float* dst, int64_t n, hipStream_t st) {
   const int64_t blocks = (n + 255) / 256;
   lm_zero_kernel<<<dim3(static_cast<unsigned>(blocks < 65536 ? blocks : 65536)), dim3(256), 0, st>>>(dst, n);

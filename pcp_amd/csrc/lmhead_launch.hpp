@@ -186,9 +186,6 @@ hipError_t launch_lm_scatter_rows(const float* src, int nsplit, int64_t stride, 
 // dst may be src.
 hipError_t launch_lm_sum_parts(const float* src, int nsplit, int64_t stride, float* dst, int64_t n, int64_t rows,
                                const int* count, hipStream_t st);
-// K pieces per tile for the fragment-major products: `tiles` tiles of `stages` 64-deep
-// stages each, in a launch whose other product adds `other` tile-stages (at all tokens).
-int lm_ksplit(int64_t tiles, int64_t stages, int64_t other);
 hipError_t launch_lm_zero(float* dst, int64_t n, hipStream_t st);
 hipError_t launch_lm_tiles(int mode, const LmTileArgs& a, hipStream_t st);
 // One launch of one or two products (n_gemm = 1 or 2; fields per LmTileArgs::Gemm,

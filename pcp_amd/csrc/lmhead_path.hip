@@ -26,7 +26,6 @@
 
 #include <hip/hip_runtime.h>
 
-#include <algorithm>
 #include <cstdint>
 #include <cstring>
 
@@ -84,6 +83,26 @@ hipError_t grow_dbuf(pcp_ctx* ctx, size_t bytes) {
   }
   ctx->lm_dbuf_bytes = want;
   return hipSuccess;
+}
+
+// Room for `bytes` of K pieces: OptionalRoom's status, or a HIP error. Like the backward
+// workspace, the pieces take at most half of the device memory that is free.
+int have_pieces(pcp_ctx* ctx, size_t bytes) {
+  static_assert(hipSuccess == static_cast<int>(OptionalRoom::kHeld), "HIP errors pass through have()");
+  auto alloc = [&](size_t want, void** p) -> int {
+    size_t free_b = 0, total_b = 0;
+    hipError_t e = hipMemGetInfo(&free_b, &total_b);
+    if (e == hipSuccess && want > (free_b + ctx->lm_pieces.bytes) / 2) return OptionalRoom::kRefused;
+    if (e == hipSuccess) e = hipMalloc(p, want);
+    if (e == hipSuccess) return OptionalRoom::kHeld;
+    (void)hipGetLastError();
+    return e == hipErrorOutOfMemory ? static_cast<int>(OptionalRoom::kRefused) : static_cast<int>(e);
+  };
+  auto retire = [](void* p) {
+    (void)hipDeviceSynchronize();
+    (void)hipFree(p);
+  };
+  return ctx->lm_pieces.have(bytes, alloc, retire);
 }
 
 int validate_lm(const pcp_lmhead_args* a) {
@@ -171,34 +190,11 @@ int run_lm(pcp_ctx* ctx, const pcp_lmhead_args* a) {
   // that one block writes or one tile reads on the same HBM channels).
   const int64_t ldt_max = (N + 63) / 64 * 64 + ((N + 63) / 64 * 64 % 256 == 0 ? 64 : 0);
   const size_t o_ht = a->dweight ? take(2 * static_cast<size_t>(H) * ldt_max) : 0;
-  // The cached backward's products in K pieces (lm_ksplit): dhidden's pieces are compact
-  // [N, H] buffers one after the other, dW's [V, H] ones. A tile's prologue and epilogue
-  // count as four stages. The pieces have room at the end for every call of up to N tokens
-  // (their number falls as N grows), so that a call of fewer tokens than the one before it
-  // needs no larger buffer; without memory for them the tiles stay whole.
-  const int64_t nht = (H + kLmTileT - 1) / kLmTileT, sd = (V + 63) / 64 + 4;
-  int split_d = 1, split_w = 1;
-  size_t d_bytes = 0, piece_bytes = 0;   // dhidden's pieces of this call; all of the largest call's
-  if (bwd && a->vocab_chunk == 0) {
-    for (int64_t s = 1; s <= (N + 63) / 64; ++s) {
-      const int64_t n = s * 64 < N ? s * 64 : N, ntk = (n + kLmTileV - 1) / kLmTileV, sw = s + 4;
-      split_d = want_dy ? lm_ksplit(ntk * nht, sd, a->dweight ? nvt * nht * sw : 0) : 1;
-      split_w = a->dweight ? lm_ksplit(nvt * nht, sw, want_dy ? ntk * nht * sd : 0) : 1;
-      d_bytes = split_d > 1 ? r256(4 * static_cast<size_t>(n) * H * split_d) : 0;
-      piece_bytes = std::max(piece_bytes, d_bytes + (split_w > 1 ? 4 * static_cast<size_t>(V) * H * split_w : 0));
-    }
-  }
-  const size_t o_dhc_whole = want_dy ? take(4 * static_cast<size_t>(N) * H) : 0;
+  const size_t o_dhc = want_dy ? take(4 * static_cast<size_t>(N) * H) : 0;
   const size_t o_rstd = norm ? take(4 * N) : 0;
   const size_t o_gpart = a->dnorm_weight ? take(4 * static_cast<size_t>(kLmNormSlices) * H) : 0;
-  const size_t whole = off, o_pieces = take(piece_bytes);
   rc = ensure_scratch(ctx, off);
-  if (rc == PCP_ERR_OOM && piece_bytes) {
-    split_d = split_w = 1;
-    rc = ensure_scratch(ctx, whole);
-  }
   if (rc != PCP_OK) return rc;
-  const size_t o_dhc = split_d > 1 ? o_pieces : o_dhc_whole, o_dwp = o_pieces + d_bytes;
   char* sp = static_cast<char*>(ctx->scratch);
   auto F = [&](size_t o) { return reinterpret_cast<float*>(sp + o); };
   auto I = [&](size_t o) { return reinterpret_cast<int*>(sp + o); };
@@ -257,6 +253,15 @@ int run_lm(pcp_ctx* ctx, const pcp_lmhead_args* a) {
                     (long long)chunk);
       return hip_fail(ctx, e, "allocating the dlogits chunk");
     }
+  }
+
+  // The cached products in K pieces; without room for them the tiles stay whole.
+  LmPieces pieces;
+  if (cached) {
+    pieces = lm_pieces(N, H, V, want_dy, a->dweight != nullptr);
+    const int have = have_pieces(ctx, lm_pieces_room(N, H, V, want_dy, a->dweight != nullptr));
+    if (have == OptionalRoom::kRefused) pieces = LmPieces{};
+    else if (have != OptionalRoom::kHeld) return hip_fail(ctx, static_cast<hipError_t>(have), "allocating the K pieces");
   }
 
   // Live-token compaction. The count stays on the device: every kernel below reads it
@@ -386,7 +391,8 @@ int run_lm(pcp_ctx* ctx, const pcp_lmhead_args* a) {
   // an empty K (dW: zero), and dead rows are written as zero, so every gradient is 0.
   if (bwd) {
     char* dbuf = static_cast<char*>(ctx->lm_dbuf);
-    float* dhc = want_dy ? F(o_dhc) : nullptr;
+    float* dhc = !want_dy ? nullptr : pieces.split_d > 1 ? static_cast<float*>(ctx->lm_pieces.buf) : F(o_dhc);
+    float* dwp = reinterpret_cast<float*>(static_cast<char*>(ctx->lm_pieces.buf) + pieces.d_bytes);
     // hidden^T [H, ldt], zero past the live tokens: an operand of dW (fragment-major
     // when it is the products' token operand on the cached path).
     const LmTransposeArgs tr{reinterpret_cast<const uint16_t*>(sp + o_hid), H, static_cast<int>(N),
@@ -481,7 +487,7 @@ int run_lm(pcp_ctx* ctx, const pcp_lmhead_args* a) {
         d.ntt = static_cast<int>((H + kLmTileT - 1) / kLmTileT);
         d.C = dhc;
         d.ldc = static_cast<int>(H);
-        d.ksplit = split_d;
+        d.ksplit = pieces.split_d;
         d.cstride = N * H;
       }
       if (a->dweight) {
@@ -499,9 +505,9 @@ int run_lm(pcp_ctx* ctx, const pcp_lmhead_args* a) {
         d.kcount = cnt;
         d.nvt = static_cast<int>((V + kLmTileV - 1) / kLmTileV);
         d.ntt = static_cast<int>((H + kLmTileT - 1) / kLmTileT);
-        d.C = split_w > 1 ? F(o_dwp) : a->dweight;
+        d.C = pieces.split_w > 1 ? dwp : a->dweight;
         d.ldc = static_cast<int>(H);
-        d.ksplit = split_w;
+        d.ksplit = pieces.split_w;
         d.cstride = V * H;
       }
       const bool timed = ctx->prof_on && ctx->prof_used < static_cast<int>(ctx->prof_start.size());
@@ -511,8 +517,8 @@ int run_lm(pcp_ctx* ctx, const pcp_lmhead_args* a) {
         return hip_fail(ctx, e, "dhidden / dweight products");
       if (timed && (e = hipEventRecord(ctx->prof_stop[ctx->prof_used++], st)) != hipSuccess)
         return hip_fail(ctx, e, "hipEventRecord");
-      if (split_w > 1 &&
-          (e = launch_lm_sum_parts(F(o_dwp), split_w, V * H, a->dweight, V * H, V, nullptr, st)) != hipSuccess)
+      if (pieces.split_w > 1 &&
+          (e = launch_lm_sum_parts(dwp, pieces.split_w, V * H, a->dweight, V * H, V, nullptr, st)) != hipSuccess)
         return hip_fail(ctx, e, "adding the dweight pieces");
     } else {
       if (a->dweight && (e = chunk_frag ? launch_lm_transpose_frag(tr, st) : launch_lm_transpose(tr, st)) != hipSuccess)
@@ -587,15 +593,15 @@ int run_lm(pcp_ctx* ctx, const pcp_lmhead_args* a) {
           return hip_fail(ctx, e, "dhidden / dweight products");
       }
     }
-    const int pieces = cached ? split_d : 1;   // of the compact dhidden
     if (norm && want_dy) {
-      if (pieces > 1 && (e = launch_lm_sum_parts(dhc, pieces, N * H, dhc, N * H, N, cnt, st)) != hipSuccess)
+      if (pieces.split_d > 1 &&
+          (e = launch_lm_sum_parts(dhc, pieces.split_d, N * H, dhc, N * H, N, cnt, st)) != hipSuccess)
         return hip_fail(ctx, e, "adding the dhidden pieces");
       const LmNormBwdArgs nb{dhc, static_cast<const uint16_t*>(a->hidden_states), a->norm_weight, F(o_rstd),
                              I(o_cidx), I(o_live), N, static_cast<int>(H), cnt, a->dhidden,
                              a->dnorm_weight ? F(o_gpart) : nullptr, a->dnorm_weight};
       if ((e = launch_lm_norm_bwd(nb, st)) != hipSuccess) return hip_fail(ctx, e, "final norm backward");
-    } else if (!norm && a->dhidden && (e = launch_lm_scatter_rows(dhc, pieces, N * H, a->dhidden, I(o_cidx),
+    } else if (!norm && a->dhidden && (e = launch_lm_scatter_rows(dhc, pieces.split_d, N * H, a->dhidden, I(o_cidx),
                                                                      static_cast<int>(N), static_cast<int>(H), st)) != hipSuccess) {
       return hip_fail(ctx, e, "scattering dhidden rows");
     }
