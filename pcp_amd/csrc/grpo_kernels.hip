@@ -977,10 +977,16 @@ __global__ void __launch_bounds__(64) grpo_part_merge_kernel(RowArgs a, int part
   write_token_outputs(a, r, static_cast<float>(lp), static_cast<float>(lr), token_terms(a, r, lp, lr).loss);
 }
 
+// f32 dlogits of 16-bit logits: a lane takes two 4-element groups 64 groups apart in place of
+// one vector, as in resident_row (kSplit), so that each store of a wave covers whole lines.
+// Storing a vector's two halves from one lane, 32 bytes between lanes, wrote every line in
+// parts through the system-scope stores: 512 rows of 151,936 took 345 us (one row to a
+// workgroup: 149), 768 rows of 50,000 199 (85); see plan_rows for the times with whole lines.
 template <typename TI, typename TO, int SP>
 __global__ void __launch_bounds__(kPartBlock) grpo_part_grad_kernel(RowArgs a, int per) {
   constexpr int EPV = 16 / TI::kBytes, U = kPartU, BLOCK = kPartBlock;
   constexpr uint32_t kOutVec = EPV * TO::kBytes;   // output bytes per input vector
+  constexpr bool kSplit = TI::kBytes == 2 && TO::kBytes == 4;
   const int tid = threadIdx.x, part = blockIdx.x;
   const int64_t row = blockIdx.y, row_elem = row * a.vocab;
   const RowMeta r = row_meta(a, row);
@@ -992,6 +998,9 @@ __global__ void __launch_bounds__(kPartBlock) grpo_part_grad_kernel(RowArgs a, i
   const uint32_t lim = static_cast<uint32_t>(end);
   const __amdgpu_buffer_rsrc_t drow =
       row_rsrc(static_cast<char*>(a.dlogits) + (row_elem + xsp.head) * TO::kBytes, lim * kOutVec);
+  // kSplit: group(q, h) is the h-th 4-element group of this lane's slot q.
+  const uint32_t sgrp = split_group<TI, TO, BLOCK>(tid);
+  auto group = [&](int q, int h) { return static_cast<uint32_t>(2 * (v0 + q * BLOCK) + 64 * h) + sgrp; };
   if (!r.live) {
     if (part == 0) write_token_outputs(a, r, 0.f, 0.f, 0.f);
     if (a.zero_fill) {
@@ -999,8 +1008,8 @@ __global__ void __launch_bounds__(kPartBlock) grpo_part_grad_kernel(RowArgs a, i
 #pragma unroll
       for (int q = 0; q < U; ++q)
 #pragma unroll
-        for (uint32_t h = 0; h < kOutVec; h += 16)
-          buf_st16<true, SP>(drow, z, static_cast<uint32_t>(v0 + q * BLOCK + tid) * kOutVec + h);
+        for (int h = 0; h < (kSplit ? 2 : 1); ++h)
+          buf_st16<true, SP>(drow, z, kSplit ? group(q, h) * 16u : static_cast<uint32_t>(v0 + q * BLOCK + tid) * 16u);
       if (ek >= 0) store1<TO>(a.dlogits, row_elem + ek, 0.f);
     }
     return;
@@ -1012,7 +1021,14 @@ __global__ void __launch_bounds__(kPartBlock) grpo_part_grad_kernel(RowArgs a, i
   const __amdgpu_buffer_rsrc_t xbuf = row_rsrc(xsp.vec, lim * 16u);
   u32x4 xb[U];
 #pragma unroll
-  for (int q = 0; q < U; ++q) xb[q] = buf_ld16<true>(xbuf, static_cast<uint32_t>(v0 + q * BLOCK + tid) * 16u);
+  for (int q = 0; q < U; ++q) {
+    if constexpr (kSplit) {
+      const u32x2 lo = buf_ld8<true>(xbuf, group(q, 0) * 8u), hi = buf_ld8<true>(xbuf, group(q, 1) * 8u);
+      xb[q] = u32x4{lo[0], lo[1], hi[0], hi[1]};
+    } else {
+      xb[q] = buf_ld16<true>(xbuf, static_cast<uint32_t>(v0 + q * BLOCK + tid) * 16u);
+    }
+  }
   const float4 mg = merge_parts(a, row, gridDim.x);
   const float lse2 = mg.x + log2f(mg.y);
   const double lse = ms_lse(mg.x, mg.y), rlse = has_ref ? ms_lse(mg.z, mg.w) : 0.;
@@ -1033,12 +1049,23 @@ __global__ void __launch_bounds__(kPartBlock) grpo_part_grad_kernel(RowArgs a, i
     float o[EPV];
 #pragma unroll
     for (int j = 0; j < EPV; ++j) o[j] = nc * hw_exp2(fmaf(TI::unpack(w, j), kLog2e, -lse2));
-    if (vi == tv) {
+    if constexpr (kSplit) {
 #pragma unroll
-      for (int j = 0; j < EPV; ++j)
-        if (j == tj) o[j] = dy;
+      for (int h = 0; h < 2; ++h) {
+        const bool mine = it >= 0 && group(q, h) == static_cast<uint32_t>(it >> 2);
+        float v[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) v[j] = mine && j == (it & 3) ? dy : o[4 * h + j];
+        buf_store_vals<TO, 4, true, SP>(drow, group(q, h) * 16u, v);
+      }
+    } else {
+      if (vi == tv) {
+#pragma unroll
+        for (int j = 0; j < EPV; ++j)
+          if (j == tj) o[j] = dy;
+      }
+      buf_store_vals<TO, EPV, true, SP>(drow, static_cast<uint32_t>(vi) * kOutVec, o);
     }
-    buf_store_vals<TO, EPV, true, SP>(drow, static_cast<uint32_t>(vi) * kOutVec, o);
   }
   if (ek >= 0)
     store1<TO>(a.dlogits, row_elem + ek, ek == r.id ? dy : nc * hw_exp2(fmaf(xe, kLog2e, -lse2)));
@@ -1464,26 +1491,38 @@ hipError_t dispatch_rows(const RowPlan& p, const RowArgs& a, const StepPrepArgs*
 
 }  // namespace
 
-// Where few rows run in parts (kParts) and not one to a workgroup. Whole calls (clip-KL,
-// half of the rows live and the rest zero-filled unless said), us, a row to a workgroup |
-// in parts:
-//   bf16 151,936  16 rows  48 | 33   64  53 | 39   256  65 | 62   512 103 |  91   768 138 | 126   1024 163 | 161   1536 218 | 227
-//   bf16 100,000                     64  46 | 37   256  51 | 54   512  80 |  74   768 103 |  97   1024 120 | 120
-//   bf16  50,257                     64  38 | 34   256  43 | 44   512  60 |  56   768  74 |  68   1024  84 |  81
-//   bf16  32,768                     64  35 | 33   256  37 | 37   512  47 |  44                   1024  62 |  56
-//   bf16  16,384                     64 32.5 | 33.4 256 32.9 | 33.5                               1024  44 |  45
-//   f32  151,936 (streamed)          64  76 | 45   256  98 | 89   512 170 | 136   768 251 | 201   1024 323 | 269   1536 456 | 417
-//   bf16 151,936, no zero-fill, a fifth live       256  58 | 42   512  59 |  51   768  61 | 60
-// (f32 151,936, REINFORCE, 2048 rows: 414 | 435.) Log-probs of policy and reference, one
+// Where few rows run in parts (kParts) and not one to a workgroup. Whole synchronous calls,
+// us, a row to a workgroup | in parts. Clip-KL, dead rows zero-filled, with all / a uniform
+// half / a fifth of the rows live:
+//   bf16 151,936   16 rows 48/48/48 | 32/32/32   64 52/54/55 | 39/38/35   256  71/ 63/ 61 |  77/ 63/ 48
+//                 512    121/104/97 | 126/96/70                           768 164/138/115 | 172/116/ 95
+//   bf16 100,000   64    44/44/44 | 37/36/34     256 55/50/49 | 62/51/46   512  92/78/76 |  93/74/60   768 123/104/88 | 122/99/78
+//   bf16  50,257   64    40/39/39 | 34/34/33     256 44/43/40 | 45/42/41   512  64/59/57 |  64/54/51   768  82/ 74/64 |  80/69/57
+//   bf16  32,768   64    36/36/36 | 34/34/33     256 38/35/36 | 37/36/36   512  52/46/44 |  46/41/42   768  63/ 54/50 |  56/49/41
+//   f32  151,936 (streamed)  64 76/77/79 | 48/44/37   512 205/175/145 | 206/147/108   1024 400/354/220 | 391/313/178
+//                          1536 603/426/317 | 577/388/253
+// The live share is not known at the launch and batches are ragged, so the line lies where
+// rows in parts still gain on average, though all-live calls lose a little. REINFORCE gains
+// less (bf16 151,936: 64 rows 42/42/42 | 35/35/33, 256 55/52/46 | 64/54/43, 512 88/77/76 |
+// 103/80/63, 768 120/100/89 | 138/96/84), calls without zero-fill with few live rows more
+// (bf16 151,936, clip-KL, a fifth live: 256 59 | 41, 512 60 | 49, 768 64 | 61).
+// f32 dlogits of 16-bit logits gain likewise from 12,000 vectors on (151,936: 64 rows
+// 57/60/54 | 41/39/36, 256 86/83/77 | 90/84/60, 512 149/131/129 | 148/115/98, 768 218/185/158 |
+// 206/161/137), narrower ones to about 96 rows only (50,000: 64 rows 38/38/38 | 34/34/33, 96
+// 39/38/38 | 38/37/36, 192 42/41/38 | 44/42/41, 512 66/62/64 | 75/65/61, 768 85/69/72 | 99/80/73).
+// Log-probs of policy and reference, one
 // workgroup of 256 lanes per row | in parts:
 //   bf16 151,936  16 rows  55 | 35   64  55 | 39   256  57 | 48   512  68 |  57   1024 100 | 88   2048 132 | 125
 //   bf16  50,257 (policy)            64  30 | 29                  512  32 |  34   1024  38 | 38   2048  48 |  44
 constexpr int64_t kPartMinVecs = 4096, kPartMaxRows = 768, kPartMaxRowsStreamed = 1536;
-constexpr int64_t kPartMinVecsFwd = 12000, kPartMaxRowsFwd = 2048;
+constexpr int64_t kPartWideVecs = 12000, kPartMaxRowsSplit = 96;
+constexpr int64_t kPartMaxRowsFwd = 2048;
 static_assert(kPartScratchBytes == sizeof(float4) * kPartMaxRowsFwd * (64 + 1), "the largest launch in parts");
 
-RowPlan plan_rows(int in_bytes, int64_t vocab, bool aligned16, bool edge_ok, bool forward_only, bool force_stream,
-                  int64_t nrows) {
+RowPlan plan_rows(const RowShape& c, int64_t nrows) {
+  const int in_bytes = c.in_bytes;
+  const int64_t vocab = c.vocab;
+  const bool aligned16 = c.aligned16, edge_ok = c.edge_ok, forward_only = c.forward_only;
   RowPlan p;
   const int epv = 16 / in_bytes;
   const bool vec = aligned16 && (vocab % epv == 0);
@@ -1494,7 +1533,7 @@ RowPlan plan_rows(int in_bytes, int64_t vocab, bool aligned16, bool edge_ok, boo
   p.edge = 0;
   p.exact = 0;
   p.parts = p.per = 0;
-  if (force_stream) return p;
+  if (c.force_stream) return p;
   const int64_t nv = vocab / epv;   // the interior of a row off 16 bytes has at most as many
   constexpr int64_t kVecs = kPartBlock * kPartU;
   auto in_parts = [&](int64_t min_vecs, int64_t max_rows) {
@@ -1506,7 +1545,7 @@ RowPlan plan_rows(int in_bytes, int64_t vocab, bool aligned16, bool edge_ok, boo
     p.per = static_cast<int>((nv + parts - 1) / parts);
     return true;
   };
-  if (forward_only && in_parts(kPartMinVecsFwd, kPartMaxRowsFwd)) return p;
+  if (forward_only && in_parts(kPartWideVecs, kPartMaxRowsFwd)) return p;
   // The forward kernel takes rows of any alignment. It addresses a row through a
   // 32-bit buffer offset that runs up to one batch past the row end: rows up to 2 GiB
   // take it, longer rows stream (64-bit addressing).
@@ -1519,7 +1558,9 @@ RowPlan plan_rows(int in_bytes, int64_t vocab, bool aligned16, bool edge_ok, boo
   // type and offset (the head and tail then line up); otherwise they stream.
   if (!vec && !edge_ok) return p;
 
-  if (!forward_only && in_parts(kPartMinVecs, kPartMaxRows)) return p;
+  if (!forward_only &&
+      in_parts(kPartMinVecs, in_bytes < c.out_bytes && nv < kPartWideVecs ? kPartMaxRowsSplit : kPartMaxRows))
+    return p;
   for (int i = 0; i < static_cast<int>(sizeof(kResCfgs) / sizeof(kResCfgs[0])); ++i) {
     if (static_cast<int64_t>(kResCfgs[i].block) * kResCfgs[i].nch >= nv) {
       p.kind = RowPlan::kResident;

@@ -21,12 +21,20 @@ struct RowPlan {
   int exact;  // bf16 -> bf16 resident rows without the f16 softmax cache (PCP_FLAG_EXACT_BF16)
 };
 
-// in_bytes: logits element size; aligned16: every row base is 16-byte aligned;
-// edge_ok: dlogits (if any) have the logits' element type and the same address mod 16,
-// so rows off 16 bytes split alike; forward_only: no dlogits are written; nrows: rows of
-// the call (of the whole call where it runs in groups: a row's bits depend on the plan).
-RowPlan plan_rows(int in_bytes, int64_t vocab, bool aligned16, bool edge_ok, bool forward_only, bool force_stream,
-                  int64_t nrows);
+// A call's rows, as far as the plan depends on them.
+struct RowShape {
+  int in_bytes;        // logits element size
+  int out_bytes;       // dlogits element size (forward_only: unused)
+  int64_t vocab;
+  bool aligned16;      // every row base is 16-byte aligned
+  bool edge_ok;        // dlogits (if any) have the logits' element type and the same address mod
+                       // 16, so rows off 16 bytes split alike
+  bool forward_only;   // no dlogits are written
+  bool force_stream;
+};
+// nrows: rows of the call (of the whole call where it runs in groups: a row's bits depend on
+// the plan).
+RowPlan plan_rows(const RowShape& shape, int64_t nrows);
 // Bytes of RowArgs::part that a plan needs for nrows rows (0 for every kind but kParts), and
 // their upper bound: 2,048 rows of 64 parts.
 constexpr size_t kPartScratchBytes = 2048 * (64 + 1) * 16;

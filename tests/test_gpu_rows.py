@@ -357,3 +357,25 @@ def test_rows_in_parts_in_place(dt, V):
     got = grpo.grpo_loss_fwd_bwd(x, ids, mask, dlogits=x, **kw)
     for f in ("loss", "dlogits", "logp", "ref_logp", "token_loss"):
         assert torch.equal(getattr(got, f), getattr(want, f)), f
+
+
+@pytest.mark.parametrize("dt", ["bf16", "f16"])
+@pytest.mark.parametrize("V", [32776, 95992, 151944])
+def test_f32_dlogits_of_16_bit_rows_in_parts(dt, V):
+    """f32 dlogits of 16-bit logits in parts against c * (onehot - softmax) in 64 bits, with targets
+    all over the row (both halves of a wave's slots, ragged last parts) and a dead row. A term is
+    one exponential of an argument below 40 in f32: 2^-24 * 40 * ln 2 of it, under 1e-5 of |c|."""
+    gen = torch.Generator(device=DEV).manual_seed(V)
+    S, T = 2, 41
+    x = (torch.randn((S, T, V), generator=gen, device=DEV) * 3).to({"bf16": torch.bfloat16, "f16": torch.float16}[dt])
+    ids = torch.linspace(0, V - 1, S * T, device=DEV).long().view(S, T)
+    mask = torch.ones((S, T), device=DEV)
+    mask[1, 7] = 0
+    adv = torch.tensor([0.75, -1.25], device=DEV)
+    out = grpo.grpo_loss_fwd_bwd(x, ids, mask, advantages=adv, dlogits=torch.full((S, T, V), 7.0, device=DEV))
+    c = (-adv.double() / (S * mask.double().sum(1)))[:, None] * mask.double()
+    want = -torch.softmax(x.double(), -1)
+    want.scatter_add_(2, ids[..., None], torch.ones_like(want[..., :1]))
+    want *= c[..., None]
+    err = (out.dlogits.double() - want).abs().amax(-1)
+    assert bool((err <= 1e-5 * c.abs()).all())
