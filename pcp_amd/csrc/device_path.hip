@@ -212,7 +212,7 @@ int run(pcp_ctx* ctx, const pcp_grpo_args* a, Op op, bool noalloc = false, int64
                                                                          reinterpret_cast<uintptr_t>(dl)) & 15u) == 0);
   auto plan_for = [&](int64_t rows) {
     RowPlan p = plan_rows({dtype_bytes(a->logits_dtype), dl ? dtype_bytes(a->dlogits_dtype) : 0, g.vocab, al, edge_ok,
-                           dl == nullptr, (a->flags & PCP_FLAG_FORCE_STREAMING) != 0}, rows);
+                           dl == nullptr, ref != nullptr, (a->flags & PCP_FLAG_FORCE_STREAMING) != 0}, rows);
     p.exact = (a->flags & PCP_FLAG_EXACT_BF16) ? 1 : 0;
     return p;
   };

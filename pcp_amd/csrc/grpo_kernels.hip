@@ -1510,14 +1510,19 @@ hipError_t dispatch_rows(const RowPlan& p, const RowArgs& a, const StepPrepArgs*
 // 57/60/54 | 41/39/36, 256 86/83/77 | 90/84/60, 512 149/131/129 | 148/115/98, 768 218/185/158 |
 // 206/161/137), narrower ones to about 96 rows only (50,000: 64 rows 38/38/38 | 34/34/33, 96
 // 39/38/38 | 38/37/36, 192 42/41/38 | 44/42/41, 512 66/62/64 | 75/65/61, 768 85/69/72 | 99/80/73).
-// Log-probs of policy and reference, one
-// workgroup of 256 lanes per row | in parts:
-//   bf16 151,936  16 rows  55 | 35   64  55 | 39   256  57 | 48   512  68 |  57   1024 100 | 88   2048 132 | 125
-//   bf16  50,257 (policy)            64  30 | 29                  512  32 |  34   1024  38 | 38   2048  48 |  44
+// Log-probs of one model, one workgroup of 256 lanes per row | in parts:
+//   bf16 151,936   16 rows 36 | 28    64 37 | 30   128 38 | 33   192 39 | 37   256 40 | 40   512  47 |  50   1024  70 |  74   2048 115 | 128
+//   f32  151,936   16      38 | 28    64 42 | 32   128 45 | 38   192 47 | 43   256 48 | 48   512  67 |  72   1024 114 | 127   2048 202 | 226
+//   f32   48,000   16      30 | 28    64 30 | 28   128 30 | 29   192 30 | 32   256 31 | 34   512  36 |  41   1024  51 |  54   2048  78 |  90
+// and of policy and reference:
+//   bf16 151,936   16 rows 54 | 35    64 54 | 39   192 57 | 51   256 58 | 57   512 76 |  78   1024 121 | 124   1536 175 | 172   2048 213 | 217
+//   bf16 100,000   16      46 | 34    64 47 | 37   192 48 | 45   256 49 | 49   512 62 |  63   1024  93 |  91   1536 130 | 121   2048 159 | 153
+//   f32  151,936   16      61 | 35    64 62 | 43   192 66 | 65   256 73 | 76   512 118 | 120  1024 209 | 212   1536 298 | 300   2048 389 | 390
 constexpr int64_t kPartMinVecs = 4096, kPartMaxRows = 768, kPartMaxRowsStreamed = 1536;
 constexpr int64_t kPartWideVecs = 12000, kPartMaxRowsSplit = 96;
-constexpr int64_t kPartMaxRowsFwd = 2048;
-static_assert(kPartScratchBytes == sizeof(float4) * kPartMaxRowsFwd * (64 + 1), "the largest launch in parts");
+constexpr int64_t kPartMaxRowsFwd = 192, kPartMaxRowsFwdRef = 1536;
+static_assert(kPartScratchBytes == sizeof(float4) * kPartMaxRowsStreamed * (64 + 1) &&
+                  kPartMaxRowsFwdRef <= kPartMaxRowsStreamed, "the largest launch in parts");
 
 RowPlan plan_rows(const RowShape& c, int64_t nrows) {
   const int in_bytes = c.in_bytes;
@@ -1545,7 +1550,7 @@ RowPlan plan_rows(const RowShape& c, int64_t nrows) {
     p.per = static_cast<int>((nv + parts - 1) / parts);
     return true;
   };
-  if (forward_only && in_parts(kPartWideVecs, kPartMaxRowsFwd)) return p;
+  if (forward_only && in_parts(kPartWideVecs, c.ref ? kPartMaxRowsFwdRef : kPartMaxRowsFwd)) return p;
   // The forward kernel takes rows of any alignment. It addresses a row through a
   // 32-bit buffer offset that runs up to one batch past the row end: rows up to 2 GiB
   // take it, longer rows stream (64-bit addressing).

@@ -30,14 +30,15 @@ struct RowShape {
   bool edge_ok;        // dlogits (if any) have the logits' element type and the same address mod
                        // 16, so rows off 16 bytes split alike
   bool forward_only;   // no dlogits are written
+  bool ref;            // the reference's rows are read too
   bool force_stream;
 };
 // nrows: rows of the call (of the whole call where it runs in groups: a row's bits depend on
 // the plan).
 RowPlan plan_rows(const RowShape& shape, int64_t nrows);
 // Bytes of RowArgs::part that a plan needs for nrows rows (0 for every kind but kParts), and
-// their upper bound: 2,048 rows of 64 parts.
-constexpr size_t kPartScratchBytes = 2048 * (64 + 1) * 16;
+// their upper bound: 1,536 rows of 64 parts.
+constexpr size_t kPartScratchBytes = 1536 * (64 + 1) * 16;
 size_t plan_part_bytes(const RowPlan& p, int64_t nrows);
 
 hipError_t launch_seq_prep(const void* mask, int mask_u8, int64_t n_seq, int64_t rows,
