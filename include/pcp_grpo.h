@@ -257,8 +257,15 @@ void pcp_free(pcp_ctx* ctx, int n_out, void** out_data, size_t* out_nbytes);
 /*
  * Device-pointer path.
  */
+/* Rows of a call: a launch with few wide rows (up to 1,536, at vocabularies of 32,768
+ * 16-bit or 16,384 f32 entries and more) deals each row to several workgroups, so the
+ * order in which a row's terms are added, and with it the last bits of its outputs, depends
+ * on the number of rows in the call and on PCP_FLAG_ASYNC (log-probs) as well as on the
+ * row's own data. With bf16 logits and dlogits such calls also round as with
+ * PCP_FLAG_EXACT_BF16. The same call gives the same bits each time. */
 /* a1: per-token log-softmax + sampled-token gather for policy (and ref if given).
- * export_qwen_forward.py:154-156 / qwen_test.mlir:257-277 (returns logp, not -logp). */
+ * export_qwen_forward.py:154-156 / qwen_test.mlir:257-277 (returns logp, not -logp).
+ * With PCP_FLAG_ASYNC the call uses no memory of the context. */
 int pcp_grpo_logprob_fwd(pcp_ctx* ctx, const pcp_grpo_args* a);
 /* a3: group-relative advantages, bit-exact with rl_shepherd.zig:462-479.
  * rewards, adv: device f32 [n]; groups are consecutive blocks of group_size (the

@@ -3,6 +3,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <atomic>
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
@@ -33,7 +34,10 @@ struct pcp_ctx {
   char last_error[512] = {};      // fixed buffer: reporting an error allocates nothing
   pcp::HostPage* page = nullptr;    // host address of the page kernels report through
   pcp::HostPage* d_page = nullptr;  // its device address
-  int* d_next_row = nullptr;     // row counter of the persistent row kernel
+  int* d_next_row = nullptr;     // row counter of the persistent row kernel (start of one allocation)
+  float4* d_loss_parts = nullptr;     // RowArgs::part of losses (same allocation)
+  float4* d_logprob_parts = nullptr;  // and of log-probs: of the synchronous call that holds
+  std::atomic<bool> logprob_parts_busy{false};   // this flag
   void* scratch = nullptr;       // per-call work buffers, grown on demand
   size_t scratch_bytes = 0;
   // Streams holding PCP_FLAG_ASYNC work (a fixed set, so recording one allocates nothing).

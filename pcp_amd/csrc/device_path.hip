@@ -7,6 +7,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <atomic>
 #include <cstdint>
 #include <cstring>
 #include <mutex>
@@ -193,6 +194,19 @@ int finish(pcp_ctx* ctx, const pcp_grpo_args* a, hipStream_t st) {
   return collect_device_errors(ctx);
 }
 
+// A context's flag, held until the call returns.
+struct PartClaim {
+  std::atomic<bool>* held = nullptr;
+  bool take(std::atomic<bool>* busy) {
+    if (busy->exchange(true, std::memory_order_acquire)) return false;
+    held = busy;
+    return true;
+  }
+  ~PartClaim() {
+    if (held) held->store(false, std::memory_order_release);
+  }
+};
+
 // noalloc: take the work buffers from the device's static scratch array instead of
 // the context's grow-only buffer (no allocation of any kind on this path).
 // plan_nrows: rows to plan for (0: the call's own).
@@ -217,22 +231,23 @@ int run(pcp_ctx* ctx, const pcp_grpo_args* a, Op op, bool noalloc = false, int64
     return p;
   };
   RowPlan plan = plan_for(plan_nrows ? plan_nrows : g.nrows);
+  // Log-probs in parts take the context's buffer for them, which only one call may use at a
+  // time. With a row to a workgroup they use no memory of the context: calls enqueued on
+  // several streams may overlap (and captured ones be replayed beside others), and so may
+  // calls of several threads.
+  PartClaim claim;
+  if (op == kLogprob && plan.kind == RowPlan::kParts &&
+      ((a->flags & PCP_FLAG_ASYNC) || !ctx || !claim.take(&ctx->logprob_parts_busy)))
+    plan = plan_for(INT64_MAX);
 
   // Scratch: adv | seq_len | seq_scale | seq_val | loss | row counter, live-row count,
-  // loss ticket | token_loss | live-row list (without zero-fill) | row parts.
+  // loss ticket | token_loss | live-row list (without zero-fill).
   const size_t sv = round256(sizeof(float) * g.n_seq);
   const bool need_tl = (op == kLoss) && a->token_loss == nullptr;
   const size_t tl_bytes = need_tl ? round256(sizeof(float) * g.n_seq * g.tstride) : 0;
   const bool need_list = (op == kLoss) && a->dlogits != nullptr && (a->flags & PCP_FLAG_NO_ZERO_FILL);
   const size_t list_bytes = need_list ? round256(sizeof(int) * static_cast<size_t>(g.nrows)) : 0;
-  size_t part_bytes = round256(plan_part_bytes(plan, g.nrows));
-  if (noalloc && 4 * sv + 512 + tl_bytes + list_bytes + part_bytes > PCP_NOALLOC_SCRATCH_BYTES) {
-    plan = plan_for(INT64_MAX);   // no room for the parts' results: a row per workgroup
-    part_bytes = 0;
-  }
-  // The context's buffer always has room for any call's parts, so that a call of fewer rows
-  // than the one before it, which may run in parts where that did not, needs no more of it.
-  const size_t need = 4 * sv + 512 + tl_bytes + list_bytes + (noalloc ? part_bytes : kPartScratchBytes);
+  const size_t need = 4 * sv + 512 + tl_bytes + list_bytes;
   if (noalloc && need > PCP_NOALLOC_SCRATCH_BYTES)
     return fail(ctx, PCP_ERR_OVERFLOW,
                 "the allocation-free call needs %zu bytes of work space, more than its %u-byte array: pass "
@@ -264,7 +279,7 @@ int run(pcp_ctx* ctx, const pcp_grpo_args* a, Op op, bool noalloc = false, int64
 
   RowArgs ra;
   std::memset(&ra, 0, sizeof(ra));
-  if (part_bytes) ra.part = reinterpret_cast<float4*>(sp + 4 * sv + 512 + tl_bytes + list_bytes);
+  if (plan.kind == RowPlan::kParts) ra.part = op == kLogprob ? ctx->d_logprob_parts : ctx->d_loss_parts;
   ra.logits = a->logits;
   ra.ids = a->ids;
   ra.mask = a->mask;
@@ -392,11 +407,17 @@ int pcp_init(int backend, int device_ordinal, pcp_ctx** out) {
   pcp_ctx* c = new (std::nothrow) pcp_ctx();
   if (!c) return fail(nullptr, PCP_ERR_OOM, "allocating the context");
   c->device = device_ordinal;
-  e = hipMalloc(&c->d_next_row, 64);
+  // The row counter, and the results of rows in parts: those of the largest call (1.6 MB), for
+  // losses and for log-probs. Held from the start, they add nothing to what a call needs.
+  void* fixed = nullptr;
+  e = hipMalloc(&fixed, 256 + 2 * kPartScratchBytes);
   if (e != hipSuccess) {
     delete c;
     return fail(nullptr, PCP_ERR_OOM, "hipMalloc(row counter): %s", hipGetErrorString(e));
   }
+  c->d_next_row = static_cast<int*>(fixed);
+  c->d_loss_parts = reinterpret_cast<float4*>(static_cast<char*>(fixed) + 256);
+  c->d_logprob_parts = c->d_loss_parts + kPartScratchBytes / sizeof(float4);
   void* page = nullptr;
   void* d_page = nullptr;
   e = hipHostMalloc(&page, sizeof(HostPage), hipHostMallocMapped | hipHostMallocCoherent);

@@ -1412,7 +1412,9 @@ hipError_t launch_fwd(const RowArgs& a, int64_t nrows, hipStream_t st) {
 template <typename TI, typename TO>
 hipError_t launch_parts(const RowPlan& p, const RowArgs& a, const StepPrepArgs* prep, int64_t nrows, hipStream_t st) {
   const int64_t nseq = prep ? prep->n_seq : 0;
-  if (nrows <= 0 || nrows != a.nrows || nrows + nseq > 65535 || a.part == nullptr || p.parts < 1 || p.parts > 64 || p.per > kPartBlock * kPartU)
+  if (nrows <= 0 || nrows != a.nrows || nrows + nseq > 65535 || a.part == nullptr ||
+      sizeof(float4) * static_cast<size_t>(nrows) * (p.parts + 1) > kPartScratchBytes || p.parts < 1 || p.parts > 64 ||
+      p.per > kPartBlock * kPartU)
     return hipErrorInvalidValue;
   const dim3 g(static_cast<unsigned>(p.parts), static_cast<unsigned>(nrows)), b(kPartBlock);
   const dim3 g1(static_cast<unsigned>(p.parts), static_cast<unsigned>(nrows + nseq));
@@ -1578,10 +1580,6 @@ RowPlan plan_rows(const RowShape& c, int64_t nrows) {
   }
   if (!forward_only) (void)in_parts(kPartMinVecs, kPartMaxRowsStreamed);
   return p;
-}
-
-size_t plan_part_bytes(const RowPlan& p, int64_t nrows) {
-  return p.kind == RowPlan::kParts ? sizeof(float4) * static_cast<size_t>(nrows) * static_cast<size_t>(p.parts + 1) : 0;
 }
 
 hipError_t launch_rows(const RowPlan& p, int in_dtype, int out_dtype, const RowArgs& a, const StepPrepArgs* prep,

@@ -36,10 +36,8 @@ struct RowShape {
 // nrows: rows of the call (of the whole call where it runs in groups: a row's bits depend on
 // the plan).
 RowPlan plan_rows(const RowShape& shape, int64_t nrows);
-// Bytes of RowArgs::part that a plan needs for nrows rows (0 for every kind but kParts), and
-// their upper bound: 1,536 rows of 64 parts.
+// Bytes of RowArgs::part (kParts), at most: 1,536 rows of 64 parts.
 constexpr size_t kPartScratchBytes = 1536 * (64 + 1) * 16;
-size_t plan_part_bytes(const RowPlan& p, int64_t nrows);
 
 hipError_t launch_seq_prep(const void* mask, int mask_u8, int64_t n_seq, int64_t rows,
                            int64_t tok_stride, int64_t tok_offset, float loss_norm,

@@ -1,6 +1,8 @@
 """Row-kernel cases the sweep does not reach: peaked bf16 rows, where the resident
 kernel's f16 softmax terms matter, and calls that leave dead rows unwritten
 (PCP_FLAG_NO_ZERO_FILL) on every row kernel. Bars: tests/parity_tol.py."""
+import threading
+
 import numpy as np
 import pytest
 import torch
@@ -379,3 +381,63 @@ def test_f32_dlogits_of_16_bit_rows_in_parts(dt, V):
     want *= c[..., None]
     err = (out.dlogits.double() - want).abs().amax(-1)
     assert bool((err <= 1e-5 * c.abs()).all())
+
+
+def test_async_logprobs_share_a_context():
+    """Log-probs enqueued on several streams through one context, beside losses and a synchronous
+    call: each gives the bits that it gives alone (they use no memory of the context)."""
+    gen = torch.Generator(device=DEV).manual_seed(4)
+    V, sizes = 151936, [150, 40, 97, 64]
+    x = [torch.randn((1, n, V), generator=gen, device=DEV).to(torch.bfloat16) for n in sizes]
+    ids = [torch.randint(0, V, (1, n), generator=gen, device=DEV) for n in sizes]
+    ctx = grpo.Context(0)
+    want = []
+    for a, i in zip(x, ids):
+        want.append(grpo.logprob_fwd(a, i, sync=False, ctx=ctx)[0])
+        ctx.sync()
+    kw = dict(advantages=torch.ones(1, device=DEV), dlogits=torch.empty_like(x[0]), ctx=ctx)
+    loss = grpo.grpo_loss_fwd_bwd(x[0], ids[0], **kw)
+    lp, dl = loss.logp.clone(), loss.dlogits.clone()
+    streams = [torch.cuda.Stream() for _ in sizes]
+    torch.cuda.synchronize()
+    for rep in range(5):
+        print(f"overlapping log-probs {rep}", flush=True)
+        with torch.cuda.stream(streams[0]):
+            loss = grpo.grpo_loss_fwd_bwd(x[0], ids[0], sync=False, **kw)
+        got = []
+        for s, a, i in zip(streams[1:], x[1:], ids[1:]):
+            with torch.cuda.stream(s):
+                got.append(grpo.logprob_fwd(a, i, sync=False, ctx=ctx)[0])
+        alone = grpo.logprob_fwd(x[3], ids[3], ctx=ctx)[0]
+        ctx.sync()
+        torch.cuda.synchronize()
+        assert all(torch.equal(g, w) for g, w in zip(got, want[1:]))
+        assert torch.equal(loss.logp, lp) and torch.equal(loss.dlogits, dl)
+        assert bool(((alone - want[3]).abs() <= 1e-5 * want[3].abs()).all())
+
+
+def test_logprobs_of_several_threads():
+    """Synchronous log-probs of two threads, each on its own stream, through one context. The
+    library's calls run outside the interpreter lock, so they overlap."""
+    gen = torch.Generator(device=DEV).manual_seed(5)
+    V, n = 151936, 96
+    x = [torch.randn((1, n, V), generator=gen, device=DEV) for _ in range(2)]
+    ids = [torch.randint(0, V, (1, n), generator=gen, device=DEV) for _ in range(2)]
+    want = [torch.log_softmax(a.double(), -1).gather(2, i[..., None])[..., 0] for a, i in zip(x, ids)]
+    ctx = grpo.Context(0)
+    torch.cuda.synchronize()
+    worst = [0.0, 0.0]
+
+    def work(k):
+        stream = torch.cuda.Stream()
+        with torch.cuda.stream(stream):
+            for _ in range(50):
+                lp, _ = grpo.logprob_fwd(x[k], ids[k], ctx=ctx)
+                worst[k] = max(worst[k], float(((lp - want[k]) / want[k]).abs().max()))
+
+    threads = [threading.Thread(target=work, args=(k,)) for k in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert max(worst) <= 1e-6

@@ -39,24 +39,30 @@ def bf16_dev(h):
     return torch.from_numpy(h.view(np.int16)).to(DEV).view(torch.bfloat16)
 
 
-def run(c, noalloc, token_loss_out, flags=0):
+def run(c, noalloc, token_loss_out, flags=0, tok_stride=0):
     """One call through the C ABI; token_loss_out False leaves token_loss NULL so the
-    library keeps the per-token losses in its work buffers. dlogits start as 7.0, so
+    library keeps the per-token losses in its work buffers. tok_stride spreads the token
+    arrays' sequences that far apart. dlogits start as 7.0, so
     rows a PCP_FLAG_NO_ZERO_FILL call leaves untouched keep that value."""
     S, T, V = c["S"], c["T"], c["V"]
+    TS = tok_stride or T
     pol, ref = bf16_dev(c["pol"]), bf16_dev(c["ref"])
-    ids = torch.from_numpy(c["ids"]).to(DEV)
-    mask = torch.from_numpy(c["mask"]).to(DEV)
+
+    def tokens(x):
+        t = torch.zeros((S, TS), dtype=torch.from_numpy(x).dtype, device=DEV)
+        t[:, :T] = torch.from_numpy(x).to(DEV)
+        return t
+
+    ids, mask, old = tokens(c["ids"]), tokens(c["mask"]), tokens(c["old"])
     rewards = torch.from_numpy(c["rewards"]).to(DEV)
-    old = torch.from_numpy(c["old"]).to(DEV)
     dl = torch.full((S, T, V), 7.0, dtype=torch.bfloat16, device=DEV)
-    logp = torch.zeros((S, T), dtype=torch.float32, device=DEV)
+    logp = torch.zeros((S, TS), dtype=torch.float32, device=DEV)
     ref_logp = torch.zeros_like(logp)
     tl = torch.zeros_like(logp) if token_loss_out else None
     adv = torch.zeros(S, dtype=torch.float32, device=DEV)
     loss = torch.zeros((), dtype=torch.float32, device=DEV)
     a = _lib.default_args()
-    grpo.fill_args(a, pol, ids, mask, T, 0, S, T, V, T)
+    grpo.fill_args(a, pol, ids, mask, T, 0, S, T, V, TS)
     a.group_size = c["G"]
     a.ref_logits = ref.data_ptr() if c["mode"] == LossMode.GRPO_CLIP_KL else None
     a.old_logp = old.data_ptr()
@@ -126,6 +132,16 @@ def test_noalloc_without_zero_fill_walks_the_listed_rows():
                             old_logp=c["old"], loss_mode=int(c["mode"]), dtype=orc.BF16)
         scale = 20.0 * float(np.abs(exp.adv).mean() * 1.5 + 0.04) + abs(exp.loss)
         assert abs(float(got["loss"]) - exp.loss) <= 1e-5 * scale, (got["loss"], exp.loss)
+
+
+@pytest.mark.parametrize("tok_stride", [0, 65000])
+@pytest.mark.parametrize("flags", [0, _lib.FLAG_NO_ZERO_FILL])
+def test_noalloc_rows_in_parts(flags, tok_stride):
+    """Few wide rows, which run in parts: the same bits from both entry points, also with token
+    arrays whose per-token losses (16 * 65,000 floats) fill the static array but for 32 KB."""
+    c = make_case(5, S=16, T=9, V=33000, G=4, mode=LossMode.GRPO_CLIP_KL)
+    print(f"noalloc rows in parts: flags={flags} tok_stride={tok_stride}", flush=True)
+    assert_same(run(c, True, False, flags, tok_stride), run(c, False, False, flags, tok_stride))
 
 
 @pytest.mark.parametrize("overflow", ["token_loss", "row_list"])
