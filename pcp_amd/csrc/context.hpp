@@ -23,7 +23,7 @@ namespace pcp {
 // every synchronous call a 4-byte hipMemcpy after its wait: see collect_device_errors.)
 struct HostPage {
   int err[8];                      // err[i] != 0: condition 1 << i (kErr* bits) was raised
-  int b64_pad;                     // padding characters of the last base64 decode
+  int b64_pad[64];                 // padding characters of a base64 decode, a slot per call in turn
   alignas(64) char stats[64];      // the gradient statistics' result
 };
 }  // namespace pcp
@@ -34,6 +34,7 @@ struct pcp_ctx {
   char last_error[512] = {};      // fixed buffer: reporting an error allocates nothing
   pcp::HostPage* page = nullptr;    // host address of the page kernels report through
   pcp::HostPage* d_page = nullptr;  // its device address
+  std::atomic<unsigned> b64_turn{0};  // base64 decodes begun: calls of several threads use different slots
   int* d_next_row = nullptr;     // row counter of the persistent row kernel (start of one allocation)
   float4* d_loss_parts = nullptr;     // RowArgs::part of losses (same allocation)
   float4* d_logprob_parts = nullptr;  // and of log-probs: of the synchronous call that holds

@@ -407,6 +407,7 @@ int pcp_base64_decode(pcp_ctx* ctx, const char* src, int64_t len, void* dst, int
   if (e != hipSuccess) return hip_fail(ctx, e, "hipSetDevice");
   if (len == 0) return PCP_OK;
   hipStream_t st = static_cast<hipStream_t>(stream);
+  const unsigned slot = ctx->b64_turn.fetch_add(1, std::memory_order_relaxed) % (sizeof(HostPage::b64_pad) / sizeof(int));
   const int64_t nq = len / 4;
   const bool aligned = (reinterpret_cast<uintptr_t>(src) & 15u) == 0 && (reinterpret_cast<uintptr_t>(dst) & 3u) == 0;
   const int64_t nunits = aligned ? (nq - 1) / 4 : 0;   // the final quad (padding) always takes the byte path
@@ -416,13 +417,13 @@ int pcp_base64_decode(pcp_ctx* ctx, const char* src, int64_t len, void* dst, int
         reinterpret_cast<const u32x4*>(src), nunits, static_cast<uint32_t*>(dst), ctx->d_page->err);
   b64_decode_quads_kernel<<<grid_for(nq - 4 * nunits, 256), 256, 0, st>>>(
       reinterpret_cast<const uint8_t*>(src), nq, 4 * nunits, static_cast<uint8_t*>(dst), ctx->d_page->err,
-      &ctx->d_page->b64_pad);
+      ctx->d_page->b64_pad + slot);
   prof_end(ctx, st, timed);
   if ((e = hipGetLastError()) != hipSuccess) return hip_fail(ctx, e, "base64 launch");
   if ((e = hipStreamSynchronize(st)) != hipSuccess) return hip_fail(ctx, e, "hipStreamSynchronize");
   const int rc = collect_device_errors(ctx);
   if (rc != PCP_OK) return rc;
-  *nbytes = nq * 3 - ctx->page->b64_pad;
+  *nbytes = nq * 3 - __atomic_load_n(ctx->page->b64_pad + slot, __ATOMIC_RELAXED);
   return PCP_OK;
 }
 

@@ -4,14 +4,16 @@ tools/prepare_rl_dataset.py, numpy tobytes as in tools/convert_weights.py) and
 Python's base64 module (the same RFC 4648 standard alphabet as std.base64.standard).
 Everything here is byte work: bit-exact."""
 import base64
+import os
 import struct
+import threading
 
 import numpy as np
 import pytest
 import torch
 
 from oracle import oracle as orc
-from pcp_amd import formats, step
+from pcp_amd import formats, grpo, step
 from pcp_amd._lib import PcpError
 
 pytestmark = pytest.mark.gpu
@@ -110,6 +112,29 @@ def test_base64_every_byte_value():
                 assert e.value.code == -1
     words = base64.b64decode(bytes(alphabet[(i + k) % 64] for k in range(16) for i in range(64)))
     assert formats.b64encode(torch.from_numpy(np.frombuffer(words, np.uint8).copy()).to(DEV)).cpu().numpy().tobytes() == base64.b64encode(words)
+
+
+def test_base64_decodes_of_several_threads():
+    """Decodes of three threads, each on its own stream with another padding, through one context:
+    each gets its own length (the library's calls run outside the interpreter lock)."""
+    ctx = grpo.Context(0)
+    raw = [os.urandom(3000 + k) for k in range(3)]
+    text = [torch.from_numpy(np.frombuffer(base64.b64encode(r), np.uint8).copy()).to(DEV) for r in raw]
+    torch.cuda.synchronize()
+    wrong = [0, 0, 0]
+
+    def work(k):
+        with torch.cuda.stream(torch.cuda.Stream()):
+            for _ in range(300):
+                got = formats.b64decode(text[k], ctx=ctx)
+                wrong[k] += got.numel() != len(raw[k]) or got.cpu().numpy().tobytes() != raw[k]
+
+    threads = [threading.Thread(target=work, args=(k,)) for k in range(3)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert wrong == [0, 0, 0]
 
 
 def test_update_weights_payload_full_size():
