@@ -483,7 +483,8 @@ __device__ __forceinline__ TokenTerms token_terms(const RowArgs& a, const RowMet
     o.loss = r.w * static_cast<float>(-lp);
     o.coef = -A * scale;
   } else {
-    const float rho = a.old_logp ? expf(static_cast<float>(lp - static_cast<double>(a.old_logp[r.tix]))) : 1.f;
+    // On-policy: 1, but NaN for a target of probability 0 (lp = -inf), as lp - lp is.
+    const float rho = expf(static_cast<float>(lp - (a.old_logp ? static_cast<double>(a.old_logp[r.tix]) : lp)));
     const float lo = 1.f - a.clip_eps, hi = 1.f + a.clip_eps;
     const float rc = fminf(fmaxf(rho, lo), hi);
     const float surr = fminf(rho * A, rc * A);

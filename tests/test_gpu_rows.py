@@ -441,3 +441,28 @@ def test_logprobs_of_several_threads():
     for t in threads:
         t.join()
     assert max(worst) <= 1e-6
+
+
+@pytest.mark.parametrize("S,T,V,kw", [(2, 6, 1000, {}), (2, 6, 5003, dict(force_streaming=True)), (2, 6, 50257, {}),
+                                      (2, 400, 33000, {})], ids=["resident", "streaming", "parts", "wide"])
+def test_target_of_probability_zero(S, T, V, kw):
+    """A live token whose own logit is -inf (masked vocabulary) on-policy: rho = exp(lp - lp) is NaN
+    for it, as in the oracle; other rows are untouched."""
+    gen = torch.Generator(device=DEV).manual_seed(6)
+    x = torch.randn((S, T, V), generator=gen, device=DEV)
+    ids = torch.randint(0, V, (S, T), generator=gen, device=DEV)
+    x[1, 2, ids[1, 2]] = -float("inf")
+    ref = x + 0.1 * torch.randn((S, T, V), generator=gen, device=DEV)
+    ref[1, 2, ids[1, 2]] = 0.0
+    adv = torch.tensor([0.5, -0.5], device=DEV)
+    out = grpo.grpo_loss_fwd_bwd(x, ids, advantages=adv, ref_logits=ref, loss_mode=LossMode.GRPO_CLIP_KL, **kw)
+    few = slice(0, 4)                                    # rows are independent: the oracle takes the first few
+    want = orc.grpo_full(x[:, few].cpu().numpy(), ids[:, few].cpu().numpy(), np.ones((S, 4), np.float32), rows=4,
+                         advantages_in=adv.cpu().numpy(), ref_logits=ref[:, few].cpu().numpy(),
+                         loss_mode=orc.CLIP_KL, dtype=orc.F32)
+    bad = np.zeros((S, T), bool)
+    bad[1, 2] = True
+    assert np.isnan(want.token_loss[1, 2]) and np.isfinite(np.delete(want.token_loss.ravel(), 4 + 2)).all()
+    assert np.array_equal(np.isnan(out.token_loss.cpu().numpy()), bad)
+    assert float(out.logp[1, 2]) == -float("inf")
+    assert np.array_equal(torch.isnan(out.dlogits).any(-1).cpu().numpy(), bad)
