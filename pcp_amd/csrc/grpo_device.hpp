@@ -389,7 +389,7 @@ struct RowArgs {
   int* row_list;
   int* row_count;
   float4* part;            // RowPlan::kParts: [nrows, parts] (policy m, s, reference m, s), then
-                           // [nrows] (the target's policy and reference logits)
+                           // [nrows] (the target's policy and reference logits, its old log-prob)
   int64_t nrows;           // logits rows of the launch
   int64_t vocab;
   int64_t rows;
@@ -467,9 +467,10 @@ struct TokenTerms {
   float coef;  // c = d loss / d logp (already includes m / (loss_norm * L_s))
 };
 
-// lp, lr: log-probs in f64, so that the differences below lose nothing of them.
-__device__ __forceinline__ TokenTerms token_terms(const RowArgs& a, const RowMeta& r, double lp,
-                                                  double lr) {
+// lp, lr: log-probs in f64, so that the differences below lose nothing of them. old():
+// the token's behaviour-policy log-prob, called only where the loss has one.
+template <typename Old>
+__device__ __forceinline__ TokenTerms token_terms(const RowArgs& a, const RowMeta& r, double lp, double lr, Old old) {
   TokenTerms o;
   if (a.adv == nullptr) {  // forward-only request: no loss terms
     o.loss = 0.f;
@@ -484,7 +485,7 @@ __device__ __forceinline__ TokenTerms token_terms(const RowArgs& a, const RowMet
     o.coef = -A * scale;
   } else {
     // On-policy: 1, but NaN for a target of probability 0 (lp = -inf), as lp - lp is.
-    const float rho = expf(static_cast<float>(lp - (a.old_logp ? static_cast<double>(a.old_logp[r.tix]) : lp)));
+    const float rho = expf(static_cast<float>(lp - (a.old_logp ? static_cast<double>(old()) : lp)));
     const float lo = 1.f - a.clip_eps, hi = 1.f + a.clip_eps;
     const float rc = fminf(fmaxf(rho, lo), hi);
     const float surr = fminf(rho * A, rc * A);
@@ -498,6 +499,10 @@ __device__ __forceinline__ TokenTerms token_terms(const RowArgs& a, const RowMet
     o.coef = scale * (dsurr - a.kl_beta * expm1f(dlr));
   }
   return o;
+}
+
+__device__ __forceinline__ TokenTerms token_terms(const RowArgs& a, const RowMeta& r, double lp, double lr) {
+  return token_terms(a, r, lp, lr, [&] { return a.old_logp[r.tix]; });
 }
 
 // Write per-token outputs of a token row (thread 0 only).

@@ -878,7 +878,8 @@ __global__ void __launch_bounds__(kSmallBlock) step_prep_kernel(StepPrepArgs a) 
 // split as in grpo_fwd_kernel, part 0 taking the head and the tail. Every dlogit is the
 // f32 result rounded once. dlogits may be the logits themselves, as with a row to a
 // workgroup: a part reads its own vectors before it writes them, and the target's logit,
-// which may lie in another part, comes from the first kernel. The first kernel, which needs neither lengths nor advantages,
+// which may lie in another part, comes from the first kernel. So does its old log-prob: part
+// 0 may write the new one over it. The first kernel, which needs neither lengths nor advantages,
 // also carries the loss's step_prep, so the loss takes no launch more than with a row to a
 // workgroup.
 // ---------------------------------------------------------------------------
@@ -941,9 +942,9 @@ __global__ void __launch_bounds__(kPartBlock) grpo_part_kernel(RowArgs a, StepPr
   block_merge2<BLOCK>(pm, ps, rm, rs, lds);
   if (tid == 0) {
     a.part[row * gridDim.x + part] = make_float4(pm, ps, rm, rs);
-    if (part == 0)   // the target's logits, which dlogits written in place may replace
-      a.part[a.nrows * gridDim.x + row] =
-          make_float4(TI::load1(xrow, r.id), REF ? TI::load1(rrow, r.id) : 0.f, 0.f, 0.f);
+    if (part == 0)   // what dlogits or log-probs written in place may replace
+      a.part[a.nrows * gridDim.x + row] = make_float4(TI::load1(xrow, r.id), REF ? TI::load1(rrow, r.id) : 0.f,
+                                                      a.old_logp ? a.old_logp[r.tix] : 0.f, 0.f);
   }
 }
 
@@ -1033,7 +1034,7 @@ __global__ void __launch_bounds__(kPartBlock) grpo_part_grad_kernel(RowArgs a, i
   const float lse2 = mg.x + log2f(mg.y);
   const double lse = ms_lse(mg.x, mg.y), rlse = has_ref ? ms_lse(mg.z, mg.w) : 0.;
   const double lp = xy - lse, lr = ry - rlse;
-  const TokenTerms tt = token_terms(a, r, lp, lr);
+  const TokenTerms tt = token_terms(a, r, lp, lr, [&] { return target.z; });
   if (part == 0) {
     flag_nonfinite(a, lse, rlse);
     write_token_outputs(a, r, static_cast<float>(lp), static_cast<float>(lr), tt.loss);

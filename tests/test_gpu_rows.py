@@ -356,6 +356,14 @@ def test_rows_in_parts_in_place(dt, V):
     kw = dict(advantages=torch.tensor([0.75, -1.25, 0.5, 1.0], device=DEV), ref_logits=ref,
               old_logp=-torch.rand((S, T), generator=gen, device=DEV) * 9, loss_mode=LossMode.GRPO_CLIP_KL)
     want = grpo.grpo_loss_fwd_bwd(x, ids, mask, dlogits=torch.empty_like(x), **kw)
+    f32 = dict(dtype=torch.float32, device=DEV)
+    # The new log-probs over the old ones.
+    over = grpo.GrpoOutputs(loss=torch.zeros((), **f32), dlogits=torch.empty_like(x), logp=kw["old_logp"].clone(),
+                            ref_logp=torch.zeros((S, T), **f32), token_loss=torch.zeros((S, T), **f32),
+                            advantages=torch.zeros(S, **f32))
+    got = grpo.grpo_loss_fwd_bwd(x, ids, mask, outputs=over, **{**kw, "old_logp": over.logp})
+    for f in ("loss", "dlogits", "logp", "ref_logp", "token_loss"):
+        assert torch.equal(getattr(got, f), getattr(want, f)), f
     got = grpo.grpo_loss_fwd_bwd(x, ids, mask, dlogits=x, **kw)
     for f in ("loss", "dlogits", "logp", "ref_logp", "token_loss"):
         assert torch.equal(getattr(got, f), getattr(want, f)), f
