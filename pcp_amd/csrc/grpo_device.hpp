@@ -390,6 +390,7 @@ struct RowArgs {
   int* row_count;
   float4* part;            // RowPlan::kParts: [nrows, parts] (policy m, s, reference m, s), then
                            // [nrows] (the target's policy and reference logits, its old log-prob)
+  int32_t turn;            // resident rows dealt in grid strides: where the next stride starts
   int64_t nrows;           // logits rows of the launch
   int64_t vocab;
   int64_t rows;

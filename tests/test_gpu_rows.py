@@ -288,6 +288,31 @@ def test_rows_past_the_first_grid(dtype, V, zero_fill, longest):
         assert torch.equal(whole[S - 4:], own)
 
 
+@pytest.mark.parametrize("T", [1, 96, 128, 509, 1024])
+@pytest.mark.parametrize("dtype, V", [("bf16", 64), ("bf16", 16384), ("f32", 1030)])
+def test_every_row_is_dealt_once(dtype, V, T):
+    """Rows dealt in grid strides that move on within the sequence: every row of calls of several
+    grids and a part comes out as in the streaming kernel, which takes a workgroup for each (to
+    2^-8 of the largest, a bf16 rounding and the f16 softmax terms; dead rows are zero in both)."""
+    dt = {"bf16": torch.bfloat16, "f32": torch.float32}[dtype]
+    S = 9001 // T
+    gen = torch.Generator(device="cuda").manual_seed(V + T)
+    x = torch.randn((S, T, V), generator=gen, device="cuda").to(dt)
+    ids = torch.randint(0, V, (S, T), generator=gen, device="cuda")
+    mask = (torch.arange(T, device="cuda")[None] < torch.randint(0, T + 1, (S, 1), generator=gen, device="cuda")).float()
+    adv = torch.rand(S, generator=gen, device="cuda") + 0.5
+
+    def call(**kw):
+        out = grpo.grpo_loss_fwd_bwd(x, ids, mask, advantages=adv, loss_norm=1.0, dlogits=torch.full_like(x, 7.0), **kw)
+        return out.dlogits.flatten(0, 1), out.logp.flatten()
+
+    got, want = call(), call(force_streaming=True)
+    assert bool(((got[1] - want[1]).abs() <= 1e-5 * want[1].abs()).all())
+    top = want[0].float().abs().amax(1)
+    assert bool(((got[0].float() - want[0].float()).abs().amax(1) <= 2 ** -8 * top).all())
+    assert bool(((mask.flatten() > 0) == (top > 0)).all())
+
+
 PARTS_CASES = [("bf16", 32768, "bf16"), ("bf16", 50257, "bf16"), ("bf16", 151936, "bf16"), ("bf16", 151937, "bf16"),
                ("bf16", 65544, "f32"), ("bf16", 262152, "bf16"), ("f32", 16384, "f32"), ("f32", 50257, "f32"),
                ("f32", 151936, "f32")]
