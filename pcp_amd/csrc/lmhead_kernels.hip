@@ -1271,6 +1271,9 @@ __global__ void __launch_bounds__(256) lm_gather_rows_kernel(const u32x4* src, u
   for (int i = threadIdx.x; i < nv; i += 256) d[i] = s[i];
 }
 
+// A result vector: 16 bytes at any element's address (dhidden and dW are the caller's).
+typedef f32x4 f32x4_any __attribute__((aligned(4)));
+
 // Element i of the sum of nsplit pieces, in order, eight loads in flight at a time.
 __device__ __forceinline__ f32x4 lm_piece_sum(const f32x4* src, int64_t i, int nsplit, int64_t stride4) {
   f32x4 acc = src[i];
@@ -1286,12 +1289,12 @@ __device__ __forceinline__ f32x4 lm_piece_sum(const f32x4* src, int64_t i, int n
   return acc;
 }
 
-__global__ void __launch_bounds__(256) lm_scatter_rows_kernel(const f32x4* src, int nsplit, int64_t stride4, f32x4* dst,
+__global__ void __launch_bounds__(256) lm_scatter_rows_kernel(const f32x4* src, int nsplit, int64_t stride4, f32x4_any* dst,
                                                               const int* cidx, int H) {
   const int t = blockIdx.x;
   const int nv = H / 4;  // 16-byte vectors per f32 row
   const int c = cidx[t];
-  f32x4* d = dst + static_cast<int64_t>(t) * nv;
+  f32x4_any* d = dst + static_cast<int64_t>(t) * nv;
   if (c >= 0) {
     const int64_t r = static_cast<int64_t>(c) * nv;
     for (int i = threadIdx.x; i < nv; i += 256) d[i] = lm_piece_sum(src, r + i, nsplit, stride4);
@@ -1301,7 +1304,7 @@ __global__ void __launch_bounds__(256) lm_scatter_rows_kernel(const f32x4* src, 
   }
 }
 
-__global__ void __launch_bounds__(256) lm_sum_parts_kernel(const f32x4* src, int nsplit, int64_t stride4, f32x4* dst,
+__global__ void __launch_bounds__(256) lm_sum_parts_kernel(const f32x4* src, int nsplit, int64_t stride4, f32x4_any* dst,
                                                            int64_t n4, int64_t row4, const int* count) {
   const int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
   if (i < n4 && (!count || i < *count * row4)) dst[i] = lm_piece_sum(src, i, nsplit, stride4);
@@ -1491,7 +1494,7 @@ hipError_t launch_lm_gather_rows(const void* src, void* dst, const int* live, co
 hipError_t launch_lm_scatter_rows(const float* src, int nsplit, int64_t stride, float* dst, const int* cidx, int N,
                                   int H, hipStream_t st) {
   lm_scatter_rows_kernel<<<dim3(N), dim3(256), 0, st>>>(reinterpret_cast<const f32x4*>(src), nsplit, stride / 4,
-                                                        reinterpret_cast<f32x4*>(dst), cidx, H);
+                                                        reinterpret_cast<f32x4_any*>(dst), cidx, H);
   return hipGetLastError();
 }
 
@@ -1499,7 +1502,7 @@ hipError_t launch_lm_sum_parts(const float* src, int nsplit, int64_t stride, flo
                                const int* count, hipStream_t st) {
   if (n <= 0 || rows <= 0) return hipSuccess;
   lm_sum_parts_kernel<<<dim3(static_cast<unsigned>((n / 4 + 255) / 256)), dim3(256), 0, st>>>(
-      reinterpret_cast<const f32x4*>(src), nsplit, stride / 4, reinterpret_cast<f32x4*>(dst), n / 4, n / rows / 4, count);
+      reinterpret_cast<const f32x4*>(src), nsplit, stride / 4, reinterpret_cast<f32x4_any*>(dst), n / 4, n / rows / 4, count);
   return hipGetLastError();
 }
 

@@ -24,6 +24,7 @@ Tolerances:
     rounding of the larger value); the target's D comes from the f32 target logit as
     without the cache.
 """
+import dataclasses
 import time
 
 import numpy as np
@@ -77,12 +78,12 @@ def oracle_case(c, mode, clip_eps=0.2, kl_beta=0.04):
 
 
 def run_device(c, mode, old, *, vocab_chunk=0, want_grads=True, ids=None, mask=None, clip_eps=0.2, kl_beta=0.04,
-               exact_bf16=False, low_memory=False):
+               exact_bf16=False, low_memory=False, outputs=None):
     return grpo.lmhead_fwd_bwd(dev(c["hb"]), dev(c["wb"]), dev(c["ids"]) if ids is None else ids,
                                dev(c["mask"]) if mask is None else mask, ref_weight=dev(c["rb"]),
                                rewards=dev(c["rewards"]), group_size=c["G"], old_logp=dev(old), loss_mode=mode,
                                clip_eps=clip_eps, kl_beta=kl_beta, vocab_chunk=vocab_chunk, want_grads=want_grads,
-                               exact_bf16=exact_bf16, low_memory_chunks=low_memory)
+                               exact_bf16=exact_bf16, low_memory_chunks=low_memory, outputs=outputs)
 
 
 def cache_error(L, lse, coef, ids):
@@ -222,6 +223,24 @@ def test_lmhead_split_products_vs_oracle(shape, exact):
     check_grads(out, *grad_bounds(c, L, lse, r, mode, old, cached=not exact))
     again = run_device(c, mode, old, exact_bf16=exact)
     assert torch.equal(out.dhidden, again.dhidden) and torch.equal(out.dweight, again.dweight)
+
+
+@pytest.mark.parametrize("off", [1, 2, 3])
+@pytest.mark.parametrize("shape", SPLIT, ids=lambda s: f"S{s[0]}T{s[1]}H{s[2]}V{s[3]}")
+def test_lmhead_split_products_unaligned_outputs(shape, off):
+    """dhidden and dweight at any element's address: the bits of the aligned buffers, and nothing
+    around them written."""
+    S, T, H, V, G, lengths = shape
+    c = make_case(S, T, H, V, G, seed=S * 977 + T + V, lengths=lengths)
+    _, _, _, old, _ = oracle_case(c, LossMode.GRPO_CLIP_KL)
+    want = run_device(c, LossMode.GRPO_CLIP_KL, old)
+    room = [torch.full((t.numel() + 8,), -3.5, device="cuda:0") for t in (want.dhidden, want.dweight)]
+    views = [r[off:off + t.numel()].view(t.shape) for r, t in zip(room, (want.dhidden, want.dweight))]
+    out = dataclasses.replace(want, dhidden=views[0], dweight=views[1])
+    got = run_device(c, LossMode.GRPO_CLIP_KL, old, outputs=out)
+    for r, g, w in zip(room, (got.dhidden, got.dweight), (want.dhidden, want.dweight)):
+        assert torch.equal(g, w)
+        assert bool((r[:off] == -3.5).all()) and bool((r[off + w.numel():] == -3.5).all())
 
 
 @pytest.mark.parametrize("shape", [s for s in SMALL if s[5] > 0], ids=lambda s: f"S{s[0]}T{s[1]}H{s[2]}V{s[3]}c{s[5]}")
