@@ -5,8 +5,9 @@ in a live row of the policy or reference logits is PCP_ERR_NONFINITE (-4). Dead 
 (mask 0) are not read for the loss, so a NaN there is not an error. After a failing call
 the error word is cleared: the next clean call succeeds and gives the clean outputs bit
 for bit. Paths: the resident kernel (bf16 and f32 logits), the streaming fallback, the
-calls without zero-fill (listed rows below half live, every row above), and the
-forward-only log-prob kernels.
+calls without zero-fill (listed rows below half live, every row above), the
+forward-only log-prob kernels, and few wide rows in parts, with the bad value in the first
+and in the last part of a row and off 16 bytes.
 """
 import numpy as np
 import pytest
@@ -18,21 +19,26 @@ from pcp_amd._lib import LossMode, PcpError
 pytestmark = pytest.mark.gpu
 
 DEV = torch.device("cuda:0")
-S, T, V = 4, 32, 4096
+S, T = 4, 32
 
 PATHS = {
-    # name: (logits dtype, sequence lengths, loss keyword arguments or None for forward-only)
-    "resident-bf16": (torch.bfloat16, [32, 20, 9, 30], {}),
-    "resident-f32": (torch.float32, [32, 20, 9, 30], {}),
-    "streaming": (torch.bfloat16, [32, 20, 9, 30], dict(force_streaming=True)),
-    "listed-no-zero-fill": (torch.bfloat16, [12, 3, 9, 7], dict(zero_fill=False)),
-    "every-row-no-zero-fill": (torch.bfloat16, [32, 20, 29, 30], dict(zero_fill=False)),
-    "logprob": (torch.bfloat16, [32, 20, 9, 30], None),
-    "logprob-streaming": (torch.bfloat16, [32, 20, 9, 30], dict(force_streaming=True, logprob=True)),
+    # name: (logits dtype, vocabulary, sequence lengths, loss keyword arguments or None for forward-only)
+    "resident-bf16": (torch.bfloat16, 4096, [32, 20, 9, 30], {}),
+    "resident-f32": (torch.float32, 4096, [32, 20, 9, 30], {}),
+    "streaming": (torch.bfloat16, 4096, [32, 20, 9, 30], dict(force_streaming=True)),
+    "listed-no-zero-fill": (torch.bfloat16, 4096, [12, 3, 9, 7], dict(zero_fill=False)),
+    "every-row-no-zero-fill": (torch.bfloat16, 4096, [32, 20, 29, 30], dict(zero_fill=False)),
+    "logprob": (torch.bfloat16, 4096, [32, 20, 9, 30], None),
+    "logprob-streaming": (torch.bfloat16, 4096, [32, 20, 9, 30], dict(force_streaming=True, logprob=True)),
+    "parts-bf16": (torch.bfloat16, 33000, [32, 20, 9, 30], {}),
+    "parts-bf16-off-16": (torch.bfloat16, 50257, [32, 20, 9, 30], {}),
+    "parts-f32": (torch.float32, 33000, [32, 20, 9, 30], {}),
+    "parts-no-zero-fill": (torch.bfloat16, 33000, [12, 3, 9, 7], dict(zero_fill=False)),
+    "logprob-parts": (torch.bfloat16, 100001, [32, 20, 9, 30], None),
 }
 
 
-def inputs(dt, lengths):
+def inputs(dt, V, lengths):
     gen = torch.Generator(device=DEV)
     gen.manual_seed(3)
     x = (torch.randn((S, T, V), generator=gen, device=DEV) * 3).to(dt)
@@ -45,7 +51,7 @@ def inputs(dt, lengths):
 
 
 def call(path, d):
-    _, _, kw = PATHS[path]
+    _, _, _, kw = PATHS[path]
     if kw is None or kw.get("logprob"):
         lp, rlp = grpo.logprob_fwd(d["x"], d["ids"], d["r"], mask=d["mask"],
                                    force_streaming=bool(kw and kw.get("force_streaming")))
@@ -62,8 +68,8 @@ def same(a, b):
 
 @pytest.mark.parametrize("path", list(PATHS))
 def test_device_errors_on_every_row_path(path):
-    dt, lengths, _ = PATHS[path]
-    d = inputs(dt, lengths)
+    dt, V, lengths, _ = PATHS[path]
+    d = inputs(dt, V, lengths)
     clean = call(path, d)
     torch.cuda.synchronize()
 
@@ -80,12 +86,17 @@ def test_device_errors_on_every_row_path(path):
     bad_ids = d["ids"].clone()
     bad_ids[2, 0] = -5                      # negative, not the ignore index
     expect(-3, "live id -5", ids=bad_ids)
+    for at in (1000, V - 1):
+        x = d["x"].clone()
+        x[0, 4, at] = float("nan")
+        expect(-4, f"NaN in a live policy row, entry {at}", x=x)
+    for at in (7, V - 2):
+        r = d["r"].clone()
+        r[3, 1, at] = float("inf")
+        expect(-4, f"+Inf in a live reference row, entry {at}", r=r)
     x = d["x"].clone()
-    x[0, 4, 1000] = float("nan")
-    expect(-4, "NaN in a live policy row", x=x)
-    r = d["r"].clone()
-    r[3, 1, 7] = float("inf")
-    expect(-4, "+Inf in a live reference row", r=r)
+    x[1, 0] = -float("inf")
+    expect(-4, "a live policy row of -Inf", x=x)
     # A NaN in a dead row (mask 0) is not read for the loss: no error, same outputs on
     # every live row (the dead row's own outputs are its fill).
     x = d["x"].clone()

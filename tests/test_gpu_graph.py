@@ -21,13 +21,16 @@ from pcp_amd._lib import LossMode
 pytestmark = pytest.mark.gpu
 
 DEV = torch.device("cuda:0")
-S, T, V, G = 16, 96, 8192, 4
+G = 4
+SHAPE = 16, 96, 8192      # sequences, rows, vocabulary
+WIDE = 8, 48, 33000        # few wide rows: in parts, whose first kernel does the step's preparation
 SENTINEL = 7.0
 
 
-def fresh_inputs(seed, dtype, lens):
+def fresh_inputs(seed, dtype, shape, lens):
     """Seeded inputs of one shape (written into the captured tensors before a replay);
     sequence lengths uniform in lens = (lo, hi)."""
+    S, T, V = shape
     gen = torch.Generator(device=DEV)
     gen.manual_seed(seed)
     pol = torch.randn((S, T, V), generator=gen, device=DEV) * 3
@@ -49,6 +52,7 @@ def call(x, out, **kw):
 
 def new_outputs(x, f32_out):
     dt = torch.float32 if f32_out else x["pol"].dtype
+    S, T, V = x["pol"].shape
     return grpo.GrpoOutputs(
         loss=torch.zeros((), dtype=torch.float32, device=DEV),
         dlogits=torch.full((S, T, V), SENTINEL, dtype=dt, device=DEV),
@@ -61,27 +65,31 @@ def new_outputs(x, f32_out):
 FIELDS = ("loss", "dlogits", "logp", "ref_logp", "token_loss", "advantages")
 
 CASES = {
-    # name: (logits dtype, f32 dlogits, zero_fill, length range, extra keyword arguments).
+    # name: (logits dtype, f32 dlogits, zero_fill, shape, length range, extra keyword arguments).
     # Without zero-fill the row kernel walks the live-row list below half live rows
     # (lengths 1..40 of 96: at most 42% live) and every row otherwise (60..96: over 62%).
-    "bf16": (torch.bfloat16, False, True, (1, T), {}),
-    "bf16-exact": (torch.bfloat16, False, True, (1, T), dict(exact_bf16=True)),
-    "bf16-f32-out": (torch.bfloat16, True, True, (1, T), {}),
-    "f32": (torch.float32, False, True, (1, T), {}),
-    "bf16-streaming": (torch.bfloat16, False, True, (1, T), dict(force_streaming=True)),
-    "bf16-nzf-listed": (torch.bfloat16, False, False, (1, 40), {}),
-    "bf16-nzf-every-row": (torch.bfloat16, False, False, (60, T), {}),
-    "bf16-noalloc-nzf-listed": (torch.bfloat16, False, False, (1, 40), dict(noalloc=True)),
-    "bf16-noalloc": (torch.bfloat16, False, True, (1, T), dict(noalloc=True)),
+    "bf16": (torch.bfloat16, False, True, SHAPE, (1, 96), {}),
+    "bf16-exact": (torch.bfloat16, False, True, SHAPE, (1, 96), dict(exact_bf16=True)),
+    "bf16-f32-out": (torch.bfloat16, True, True, SHAPE, (1, 96), {}),
+    "f32": (torch.float32, False, True, SHAPE, (1, 96), {}),
+    "bf16-streaming": (torch.bfloat16, False, True, SHAPE, (1, 96), dict(force_streaming=True)),
+    "bf16-nzf-listed": (torch.bfloat16, False, False, SHAPE, (1, 40), {}),
+    "bf16-nzf-every-row": (torch.bfloat16, False, False, SHAPE, (60, 96), {}),
+    "bf16-noalloc-nzf-listed": (torch.bfloat16, False, False, SHAPE, (1, 40), dict(noalloc=True)),
+    "bf16-noalloc": (torch.bfloat16, False, True, SHAPE, (1, 96), dict(noalloc=True)),
+    "parts-bf16": (torch.bfloat16, False, True, WIDE, (1, 48), {}),
+    "parts-f32": (torch.float32, False, True, WIDE, (1, 48), {}),
+    "parts-nzf": (torch.bfloat16, False, False, WIDE, (1, 48), {}),
+    "parts-noalloc": (torch.bfloat16, False, True, WIDE, (1, 48), dict(noalloc=True)),
 }
 
 
 @pytest.mark.parametrize("case", list(CASES))
 def test_loss_graph_capture_replays(case):
-    dtype, f32_out, zero_fill, lens, kw = CASES[case]
+    dtype, f32_out, zero_fill, shape, lens, kw = CASES[case]
     kw = dict(kw, zero_fill=zero_fill)
     ctx = grpo.default_context(0)
-    x = fresh_inputs(100, dtype, lens)
+    x = fresh_inputs(100, dtype, shape, lens)
     out = new_outputs(x, f32_out)
     call(x, out, **kw)                        # grows the work buffer; warms the launch caches
     torch.cuda.synchronize()
@@ -90,7 +98,7 @@ def test_loss_graph_capture_replays(case):
         call(x, out, sync=False, ctx=ctx, **kw)
     ctx.sync()
     for rep in range(3):
-        y = fresh_inputs(200 + rep, dtype, lens)
+        y = fresh_inputs(200 + rep, dtype, shape, lens)
         for k in x:
             x[k].copy_(y[k])
         want = new_outputs(x, f32_out)

@@ -41,13 +41,15 @@ def peaked_case(V, S, T, seed):
     return orc.bf16_from_f32(x), orc.bf16_from_f32(ref), ids, mask, rewards
 
 
-@pytest.mark.parametrize("V,S,T", [(1000, 8, 16), (151936, 4, 8)])
-def test_peaked_bf16_rows(V, S, T):
+@pytest.mark.parametrize("V,S,T,among", [(1000, 8, 16, 8), (151936, 4, 8, 4), (151936, 4, 8, 100)])
+def test_peaked_bf16_rows(V, S, T, among):
     """Two near-tied dominant logits per row (p ~ 0.3-0.5 each) in one lane. By default
     the kernel's f16 softmax terms carry up to 2^-11 of these large dlogits, inside the
     cached bar; with PCP_FLAG_EXACT_BF16 every output is the f32 result rounded once,
     inside the exact bar. Where the term is in f16's normal range (|d| >= 2^-14 |c|) the
-    two differ by at most one bf16 ulp, since 2^-11 of a value is under half its ulp."""
+    two differ by at most one bf16 ulp, since 2^-11 of a value is under half its ulp. The
+    case's S sequences are the first of `among`, the others masked: with few wide rows both
+    calls run in parts, which have no f16 terms, so the widest instance needs the 800 rows."""
     x, ref, ids, mask, rewards = peaked_case(V, S, T, seed=V + S)
     G = 2
     sel = np.ascontiguousarray(x).reshape(S * T, V)
@@ -63,14 +65,19 @@ def test_peaked_bf16_rows(V, S, T):
     ts = token_scale(x, ids, T, 0, orc.BF16)
     fl = tok_to_rows(full_floor(want, mask, old, S, False, 0.04, 0.2, ts), T, 0, T)
     bits = {}
+
+    def all_rows(a):
+        a = dev(a)
+        return torch.cat([a, torch.zeros((among - S, *a.shape[1:]), dtype=a.dtype, device=DEV)])
+
     for exact in (False, True):
-        print(f"peaked bf16 rows: V={V} S={S} T={T} exact={exact}", flush=True)
-        out = grpo.grpo_loss_fwd_bwd(dev(x), dev(ids), dev(mask), rewards=dev(rewards), group_size=G,
-                                     ref_logits=dev(ref), old_logp=dev(old), loss_mode=LossMode.GRPO_CLIP_KL,
-                                     exact_bf16=exact)
+        print(f"peaked bf16 rows: V={V} S={S} T={T} among {among} exact={exact}", flush=True)
+        out = grpo.grpo_loss_fwd_bwd(all_rows(x), all_rows(ids), all_rows(mask), rewards=all_rows(rewards), group_size=G,
+                                     ref_logits=all_rows(ref), old_logp=all_rows(old), loss_norm=float(S),
+                                     loss_mode=LossMode.GRPO_CLIP_KL, exact_bf16=exact)
         torch.cuda.synchronize()
-        assert np.all(np.abs(out.logp.cpu().numpy() - want.lp) <= 1e-5 * ts)
-        bits[exact] = host_bits(out.dlogits)
+        assert np.all(np.abs(out.logp[:S].cpu().numpy() - want.lp) <= 1e-5 * ts)
+        bits[exact] = host_bits(out.dlogits[:S])
         got = orc.bf16_to_f32(bits[exact])
         assert_dlogits(got, want.dlogits, fl, True, exact=exact)
         err = np.abs(got.astype(np.float64) - want.dlogits)
@@ -88,6 +95,8 @@ def test_peaked_bf16_rows(V, S, T):
     same_sign = (a >> 15) == (b >> 15)
     ulps = np.abs((a & 0x7FFF) - (b & 0x7FFF))
     assert np.all(same_sign[normal] | (ulps[normal] == 0)) and ulps[normal].max() <= 1
+    in_parts = V >= 32768 and among * T <= 768
+    assert in_parts == bool((a == b).all())
     print(f"  cached vs exact: {np.mean(ulps[normal] != 0):.2%} of normal-range elements one ulp apart", flush=True)
 
 
@@ -161,15 +170,16 @@ def test_no_zero_fill_leaves_dead_rows(kind, dt, V, odt, stream, shifted, live):
 
 
 # (logits dtype, V, dlogits dtype): aligned rows, several listed rows per workgroup
-LISTED_CASES = [("bf16", 32768, "bf16"), ("bf16", 32768, "f32"), ("f32", 8192, "f32")]
+LISTED_CASES = [("bf16", 32768, "bf16"), ("bf16", 32768, "f32"), ("f32", 8192, "f32"), ("f32", 10000, "f32")]
 
 
 @pytest.mark.parametrize("dt,V,odt", LISTED_CASES, ids=[f"{c[0]}-{c[1]}-{c[2]}" for c in LISTED_CASES])
 def test_no_zero_fill_listed_rows_prefetch(dt, V, odt):
     """Without zero-fill and a quarter of the rows live, the resident kernel walks the
     listed live rows, several per workgroup here, loading each next row's policy chunks
-    during the current row's dlogits pass (on 1024-lane instances of 2 and 4 chunks and
-    the split-half bf16 -> f32 instance). Every live row against the oracle, dead rows
+    during the current row's dlogits pass (on 1024-lane instances of 4 chunks, whose rows
+    are claimed from the counter, the 256-lane instance of 8, whose rows are dealt in
+    strides, and the split-half bf16 -> f32 instance). Every live row against the oracle, dead rows
     untouched bit for bit."""
     rng = np.random.default_rng(V + len(dt) + len(odt))
     S, T, G = 16, 512, 4
@@ -211,13 +221,14 @@ def test_no_zero_fill_listed_rows_prefetch(dt, V, odt):
 # Live-row counts around the persistent grid's size (one workgroup per resident slot,
 # a few hundred to about a thousand here): none, one, fewer than the grid, between one
 # and two grids (the second rows come from the first claim, not the counter), more,
-# and either side of the switch to visiting every row (half of 8192 rows).
+# and either side of the switch to visiting every row (half of 8192 rows). At V = 4096
+# the rows past the first grid are dealt in strides; bf16 20,000 and f32 10,000 claim them.
 LIVE_COUNTS = [0, 1, 37, 255, 256, 257, 511, 512, 513, 767, 1023, 1024, 1025, 1537, 2049, 4095, 4096]
 
 
-@pytest.fixture(scope="module")
-def count_inputs():
-    S, T, V = 16, 512, 4096
+@pytest.fixture(scope="module", params=[4096, 20000])
+def count_inputs(request):
+    S, T, V = 16, 512, request.param
     gen = torch.Generator(device=DEV)
     gen.manual_seed(77)
     x = torch.randn((S, T, V), generator=gen, device=DEV) * 3
@@ -225,8 +236,13 @@ def count_inputs():
     ids = torch.randint(0, V, (S, T), generator=gen, device=DEV)
     old = torch.randn((S, T), generator=gen, device=DEV) * 0.05 - float(np.log(V))
     rewards = torch.rand((S,), generator=gen, device=DEV)
-    return dict(S=S, T=T, V=V, x={"bf16": x.to(torch.bfloat16), "f32": x}, r={"bf16": r.to(torch.bfloat16), "f32": r},
-                ids=ids, old=old, rewards=rewards)
+    if V > 4096:
+        W = V // 2
+        return dict(S=S, T=T, V={"bf16": V, "f32": W}, x={"bf16": x.to(torch.bfloat16), "f32": x[..., :W].contiguous()},
+                    r={"bf16": r.to(torch.bfloat16), "f32": r[..., :W].contiguous()}, ids=ids % W, old=old,
+                    rewards=rewards)
+    return dict(S=S, T=T, V={"bf16": V, "f32": V}, x={"bf16": x.to(torch.bfloat16), "f32": x},
+                r={"bf16": r.to(torch.bfloat16), "f32": r}, ids=ids, old=old, rewards=rewards)
 
 
 @pytest.mark.parametrize("dt", ["bf16", "f32"])
@@ -237,7 +253,7 @@ def test_no_zero_fill_live_counts(count_inputs, n_live, dt):
     the zero-fill call's outputs bit for bit on live rows and leaves every dead row's
     dlogits as they were."""
     c = count_inputs
-    S, T, V = c["S"], c["T"], c["V"]
+    S, T, V = c["S"], c["T"], c["V"][dt]
     rng = np.random.default_rng(1000 + n_live)
     flat = np.zeros(S * T, np.float32)
     flat[rng.choice(S * T, size=n_live, replace=False)] = 1.0
@@ -315,7 +331,7 @@ def test_every_row_is_dealt_once(dtype, V, T):
 
 PARTS_CASES = [("bf16", 32768, "bf16"), ("bf16", 50257, "bf16"), ("bf16", 151936, "bf16"), ("bf16", 151937, "bf16"),
                ("bf16", 65544, "f32"), ("bf16", 262152, "bf16"), ("f32", 16384, "f32"), ("f32", 50257, "f32"),
-               ("f32", 151936, "f32")]
+               ("f32", 151936, "f32"), ("f16", 50257, "f16"), ("f16", 32776, "f32")]
 
 
 @pytest.mark.parametrize("zero_fill", [True, False])
@@ -330,7 +346,8 @@ def test_few_rows_in_parts_and_many_whole(dt, V, odt, zero_fill):
     rows, off = T - 1, 1
     x32 = rng.standard_normal((S, T, V)).astype(np.float32) * 3
     r32 = x32 + rng.standard_normal((S, T, V)).astype(np.float32) * 0.1
-    x, ref, code = (x32, r32, orc.F32) if dt == "f32" else (orc.bf16_from_f32(x32), orc.bf16_from_f32(r32), orc.BF16)
+    to, code = {"f32": (np.float32, orc.F32), "f16": (np.float16, orc.F16), "bf16": (orc.bf16_from_f32, orc.BF16)}[dt]
+    x, ref = (a.copy() if dt == "f32" else to(a) for a in (x32, r32))
     ids = rng.integers(0, V, size=(S, T)).astype(np.int64)
     ids[0, 1:] = [0, V - 1, V // 2, 7]
     ids[1, 2] = -100
@@ -346,7 +363,7 @@ def test_few_rows_in_parts_and_many_whole(dt, V, odt, zero_fill):
     fl = tok_to_rows(full_floor(want, mask, old, S, False, 0.04, 0.2, ts), rows, off, T)
     dead = np.ones((S, T), bool)
     dead[:, :rows] = (mask[:, 1:] == 0) | (ids[:, 1:] == -100)
-    tdt = {"bf16": torch.bfloat16, "f32": torch.float32}[odt]
+    tdt = {"bf16": torch.bfloat16, "f16": torch.float16, "f32": torch.float32}[odt]
 
     def padded(a, n):   # n - S sequences of masked tokens after the case's own
         a = dev(a)
@@ -363,7 +380,7 @@ def test_few_rows_in_parts_and_many_whole(dt, V, odt, zero_fill):
                                                                        0.04, S)
         bits = host_bits(out.dlogits[:S])
         got = orc.bf16_to_f32(bits) if odt == "bf16" else bits
-        assert_dlogits(got[~dead], want.dlogits[~dead], fl[~dead], odt == "bf16", exact=n == S)
+        assert_dlogits(got[~dead], want.dlogits[~dead], fl[~dead], odt != "f32", exact=n == S, f16_out=odt == "f16")
         fill = 0.0 if zero_fill else -3.5
         assert np.all(got[dead] == fill) and bool((dl[S:] == fill).all())
 
@@ -499,3 +516,26 @@ def test_target_of_probability_zero(S, T, V, kw):
     assert np.array_equal(np.isnan(out.token_loss.cpu().numpy()), bad)
     assert float(out.logp[1, 2]) == -float("inf")
     assert np.array_equal(torch.isnan(out.dlogits).any(-1).cpu().numpy(), bad)
+
+
+@pytest.mark.parametrize("V,lo,hi", [(50257, 0, 17000), (50257, 33000, 50257), (33000, 11000, 22000), (33000, 0, 32999)])
+@pytest.mark.parametrize("dt", ["bf16", "f32"])
+def test_rows_in_parts_with_masked_vocabulary(dt, V, lo, hi):
+    """A whole part of a row at -inf (with the row's head or tail off 16 bytes), and all of it but
+    one entry: log-probs and dlogits against 64 bits, zeros where the probability is."""
+    gen = torch.Generator(device=DEV).manual_seed(V + lo)
+    x = torch.randn((2, 9, V), generator=gen, device=DEV).to({"bf16": torch.bfloat16, "f32": torch.float32}[dt])
+    x[0, 2, lo:hi] = -float("inf")
+    ids = torch.randint(0, V, (2, 9), generator=gen, device=DEV)
+    ids[0, 2] = hi if hi < V else 5
+    adv = torch.tensor([0.75, -1.25], device=DEV)
+    out = grpo.grpo_loss_fwd_bwd(x, ids, advantages=adv)
+    lp = torch.log_softmax(x.double(), -1)
+    want_lp = lp.gather(2, ids[..., None])[..., 0]
+    assert bool(((out.logp - want_lp).abs() <= 1e-6 * want_lp.abs().clamp(min=1)).all())
+    want = lp.exp().neg()
+    want.scatter_add_(2, ids[..., None], torch.ones_like(want[..., :1]))
+    want *= -adv.double()[:, None, None] / (2 * 9)
+    rel = 2.0 ** -8 if dt == "bf16" else 2.0 ** -16
+    assert bool(((out.dlogits.double() - want).abs() <= rel * want.abs() + 1e-7).all())
+    assert bool((out.dlogits[0, 2, lo:hi] == 0).all())
