@@ -4,7 +4,7 @@ array helpers (shared by the logits-input and the fused LM-head tests).
   log-probs, token losses (f32 math):  |d| <= 1e-5 * max(1, |lse|)      (rel 1e-5 of the row scale)
   loss:                                the log-prob bar propagated through dloss/dlogp and
                                        dloss/dref, plus 1e-5 of the sum of |contributions|
-  dlogits, f32 output:                 |d| <= 1e-4 (north star) and <= 1e-5*|exact| + floor_row
+  dlogits, f32 output:                 |d| <= 1e-4 and <= 1e-5*|exact| + floor_row
   dlogits, bf16 output:                |d| <= (2^-8 + 2^-11 + 1.3e-5)*|exact| + (1 + 2^-6)*floor_row
   dlogits, bf16 output, exact mode:    |d| <= (2^-8 + 1.1e-5)*|exact| + (1 + 2^-7)*floor_row
 floor_row (coef_floor) is what the f32 log-prob error allows in the row's
