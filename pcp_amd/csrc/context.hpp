@@ -114,7 +114,7 @@ int collect_device_errors(pcp_ctx* ctx);
 
 // Record a stream that holds PCP_FLAG_ASYNC work for pcp_sync. When the fixed set is
 // full the stream is synchronised at once instead (its errors still reach pcp_sync
-// through the error word).
+// through the page).
 int add_pending(pcp_ctx* ctx, hipStream_t st);
 
 // pcp_grpo_loss_fwd_bwd with the row kernel planned for a call of plan_nrows rows, of

@@ -293,7 +293,7 @@ int run_loss_groups(pcp_ctx* ctx, const pcp_grpo_args& full, const In& L, const 
     e = launch_loss_reduce(tl, S, full.rows, T, full.tok_offset, slen, adv, full.loss_mode == PCP_LOSS_REINFORCE,
                            gtot, sval, full.loss, run);
   if (e != hipSuccess) return hip_fail(ctx, e, "loss reduction launch");
-  if ((rc = pcp_sync(ctx)) != PCP_OK) return rc;   // the compute stream and the device error word
+  if ((rc = pcp_sync(ctx)) != PCP_OK) return rc;   // the compute stream and the device errors
   e = hipStreamSynchronize(down);
   return e == hipSuccess ? PCP_OK : hip_fail(ctx, e, "device-to-host copy");
 }

@@ -85,7 +85,7 @@ __device__ __forceinline__ void load_block(__amdgpu_buffer_rsrc_t r, const void*
 // rotation of a 16-lane row, xor 4 a mirrored half row with its quads reversed, 2 and 1
 // quad permutations. Both passes are chains of such reductions between their few loads:
 // as ds_bpermute shuffles, with the row's uniform loaded only after the scan, a synchronous
-// call took 33.6 us in place of 31.7 at 64 rows of 151,936 f32, 27.3 in place of 26.1 at one.
+// call took 32.6 us in place of 31.4 at 64 rows of 151,936 f32, 25.1 in place of 23.9 at one.
 __device__ __forceinline__ float wave_sum(float v) {
   auto add = [](auto p) { return __uint_as_float(p[0]) + __uint_as_float(p[1]); };
   v = add(__builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false));
